@@ -82,7 +82,7 @@ def build_cpp_tests() -> Path:
 def build_oracle() -> None:
     make = shutil.which("make") or "make"
     _run([make, "-s", "-C", ROOT / "oracle", "all"])
-    if REFERENCE_TREE.is_dir():
+    if (REFERENCE_TREE / "G4HepEm").is_dir():
         _run([make, "-s", "-j8", "-C", ROOT / "oracle", "ref", f"REF={REFERENCE_TREE}"])
 
 
