@@ -921,8 +921,10 @@ __device__ void InteractTileChunk(const DevTables<R>& T, uint64_t seed, hepem_tr
   else GammaInteract<R>(T, seed, out, res, n, i, r, c);
 }
 
+// Held to 4 waves per SIMD: left alone the FP64 form takes 139 VGPRs (3 waves);
+// at 127 nothing spills.
 template <typename R>
-__global__ void __launch_bounds__(kBlock) k_interact_tiles(DevTables<R> T, uint64_t seed, hepem_tracks out, hepem_step_out res,
+__global__ void __launch_bounds__(kBlock, 4) k_interact_tiles(DevTables<R> T, uint64_t seed, hepem_tracks out, hepem_step_out res,
                                                            const uint8_t* __restrict__ code, const Staged* __restrict__ st,
                                                            const uint16_t* __restrict__ tlist,
                                                            const uint32_t* __restrict__ tinfo) {
@@ -1156,7 +1158,7 @@ __device__ void InteractBatchedTile(const DevTables<R>& T, uint64_t seed, const 
 }
 
 template <typename R, int TI>
-__global__ void __launch_bounds__(kBlock) k_interact_tiles_batched(DevTables<R> T, uint64_t seed, const BatchDev* __restrict__ d,
+__global__ void __launch_bounds__(kBlock, 4) k_interact_tiles_batched(DevTables<R> T, uint64_t seed, const BatchDev* __restrict__ d,
                                                                    const uint32_t* __restrict__ tbatch, uint32_t ntiles,
                                                                    const uint8_t* __restrict__ code,
                                                                    const Staged* __restrict__ st,
