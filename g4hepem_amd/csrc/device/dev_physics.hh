@@ -291,7 +291,7 @@ template <typename R> HD R UMSCSimpleScattering(R xmeanth, R x2meanth, Rng& rng)
   const R a = (R)1. + (R)4. * dum0 / dum1;
   const R prob = ((R)2. + a) * xmeanth / a;
   R r[2];
-  rng.flatArray(2, r);
+  rng.flatArray2(r);
   return (r[0] < prob) ? (R)-1. + (R)2. * vpow(r[1], (R)1. / ((R)1. + a)) : (R)-1. + (R)2. * r[1];
 }
 
@@ -382,7 +382,7 @@ HD R UMSCSampleCosineTheta(const DevTables<R>& T, int imat, R pStep, R preEkin, 
   const R prob = f2x0 / (f1x0 + f2x0);
   const R qprb = xmeanth / (prob * xmean1 + ((R)1. - prob) * xmean2);
   R r[3];
-  rng.flatArray(3, r);
+  rng.flatArray3(r);
   if (r[0] < qprb) {
     if (r[1] < prob) return (R)1. + vlog(dumEa + r[2] / dumEaa) * thex;
     const R var0 = ((R)1.0 - dd) * r[2];
@@ -400,7 +400,7 @@ template <typename R> HD void UMSCSampleDisplacement(R pStep, R thePhi, Msc<R>& 
   const R cbeta = (R)2.16;
   const R cbeta1 = (R)1. - vexp(-cbeta * (R)kPi);
   R rr[2];
-  rng.flatArray(2, rr);
+  rng.flatArray2(rr);
   const R psi = -vlog((R)1. - rr[0] * cbeta1) / cbeta;
   const R phi = (rr[1] < (R)0.5) ? thePhi + psi : thePhi - psi;
   R sinPhi, cosPhi;
@@ -509,7 +509,7 @@ template <typename R> HD R SampleCostModifiedTsai(R primEkin, Rng& rng) {  // .i
   const R uMax = (R)2.0 * ((R)1.0 + primEkin * (R)kInvElectronMassC2);
   R r[3], u;
   do {
-    rng.flatArray(3, r);
+    rng.flatArray3(r);
     const R uu = -vlog(r[0] * r[1]);
     u = ((R)0.25 > r[2]) ? uu * (R)1.6 : uu * (R)0.533333333;
   } while (u > uMax);
@@ -568,7 +568,7 @@ template <typename R> HD R SampleETransferMoller(R elCut, R primEkin, Rng& rng) 
   const R gf = (R)1.0 - gg * xmax + xmax * xmax * ((R)1.0 - gg + ((R)1.0 - gg * y) / (y * y));
   R dum, r[2], delta;
   do {
-    rng.flatArray(2, r);
+    rng.flatArray2(r);
     delta = xminmax / (xmin * ((R)1.0 - r[0]) + xmax * r[0]);
     const R xx = (R)1.0 - delta;
     dum = (R)1.0 - gg * delta + delta * delta * ((R)1.0 - gg + ((R)1.0 - gg * xx) / (xx * xx));
@@ -588,7 +588,7 @@ template <typename R> HD R SampleETransferBhabha(R elCut, R primEkin, Rng& rng) 
   const R gf = (R)1.0 + (xmax2 * b4 - xmin * xmin * xmin * b3 + xmax2 * b2 - xmin * b1) * beta2;
   R dum, r[2], delta;
   do {
-    rng.flatArray(2, r);
+    rng.flatArray2(r);
     delta = xminmax / (xmin * ((R)1.0 - r[0]) + xmax * r[0]);
     const R xx = delta * delta;
     dum = (R)1.0 + (xx * xx * b4 - delta * xx * b3 + xx * b2 - delta * b1) * beta2;
@@ -709,7 +709,7 @@ HD R SampleETransferSB(const DevTables<R>& T, double primEkinD, R lEkin, int imc
   const R dielSupConst = (R)T.matDensCor[imat] * primETot * primETot;
   R suppression, r[2], eGamma;
   do {
-    rng.flatArray(2, r);
+    rng.flatArray2(r);
     R kappa;
     if (!isSimply) {
       const R cumRV = r[0] * ((R)1.0 - minV) + minV;
@@ -770,7 +770,7 @@ HD R SampleETransferRB(const DevTables<R>& T, double primEkinD, R lEkin, int imc
   const R xrange = vlog(primEkin * primEkin + densityCorr) - xmin;
   R r[2], eGamma, funcVal;
   do {
-    rng.flatArray(2, r);
+    rng.flatArray2(r);
     eGamma = dsqrt(tmax(vexp(xmin + r[0] * xrange) - densityCorr, (R)0.0));
     const R y = eGamma / primTotalE;
     const R onemy = (R)1. - y;
@@ -879,7 +879,7 @@ template <typename R> HD void AnnihilateInFlight(Trk<R>& t, SecList<R>& sl, Rng&
   const R tau4 = tau2 * tau2;
   R eps, rfunc, r[2];
   do {
-    rng.flatArray(2, r);
+    rng.flatArray2(r);
     eps = epsmin * vexp(vlog(epsqot) * r[0]);
     rfunc = (R)1. - eps + ((R)2. * gam * eps - (R)1.) / (eps * tau4);
   } while (rfunc < r[1]);
@@ -1169,11 +1169,46 @@ template <typename R> HD int ElectronSelectDiscrete(const DevTables<R>& T, Trk<R
   return iDProc;
 }
 
+// Samples the interaction lengths that are used up (nial <= 0), one draw each
+// in process order (G4HepEmElectronManager.icc:36-41). A lane that needs c of
+// them takes the next c draws whichever the processes are, so the draws and
+// their logarithms are made once, in draw order, and handed out: the second
+// block and the logarithms beyond the first run only where a lane of the wave
+// needs two or more (a fresh track needs four, one that interacted in its last
+// step a single one), and they do not wait for one another.
+template <typename R> HD void SampleNumIALeft(R* nial, Rng& rng) {
+  const bool n0 = nial[0] <= (R)0., n1 = nial[1] <= (R)0., n2 = nial[2] <= (R)0., n3 = nial[3] <= (R)0.;
+  const uint32_t c1 = n0 ? 1u : 0u, c2 = c1 + (n1 ? 1u : 0u), c3 = c2 + (n2 ? 1u : 0u), cnt = c3 + (n3 ? 1u : 0u);
+  if (cnt == 0u) return;
+  const bool odd = (rng.ctr & 1u) != 0;
+  const uint32_t nb = (rng.ctr + 1u) >> 1;
+  double v0, v1;
+  rng.block(nb, v0, v1);
+  const R l0 = -vlog((R)(odd ? rng.hold : v0));
+  R l1 = l0, l2 = l0, l3 = l0;
+  double hold = v1;
+  if (cnt > 1u) {
+    double w0, w1;
+    rng.block(nb + 1u, w0, w1);
+    l1 = -vlog((R)(odd ? v0 : v1));
+    l2 = -vlog((R)(odd ? v1 : w0));
+    l3 = -vlog((R)(odd ? w0 : w1));
+    hold = cnt <= (odd ? 2u : 1u) ? v1 : w1;
+  }
+  rng.hold = hold;
+  rng.ctr += cnt;
+  // (selects, as in ResetNumIALeft: conditional stores would put nial in scratch)
+  const R k2 = c2 == 0u ? l0 : (c2 == 1u ? l1 : l2);
+  const R k3 = c3 == 0u ? l0 : (c3 == 1u ? l1 : (c3 == 2u ? l2 : l3));
+  nial[0] = n0 ? l0 : nial[0];
+  nial[1] = n1 ? (c1 ? l1 : l0) : nial[1];
+  nial[2] = n2 ? k2 : nial[2];
+  nial[3] = n3 ? k3 : nial[3];
+}
+
 // G4HepEmElectronManager::HowFar(data, pars, tlData) (:35-45, 166-169)
 template <typename R> HD void ElectronHowFar(const DevTables<R>& T, ElState<R>& el, Rng& rng) {
-#pragma unroll
-  for (int ip = 0; ip < 4; ++ip)
-    if (el.t.nial[ip] <= (R)0.) el.t.nial[ip] = -vlog((R)rng.flat());
+  SampleNumIALeft(el.t.nial, rng);
   HowFarToDiscreteInteraction(T, el);
   HowFarToMSC(T, el, rng);
 }
@@ -1277,7 +1312,7 @@ template <typename R> HD void ComptonPerform(Trk<R>& t, SecList<R>& sl, Rng& rng
   const R al2 = al1 + (R)0.5 * ((R)1. - eps02);
   R eps, eps2, gf, oneMinusCost, sint2, r[3];
   do {
-    rng.flatArray(3, r);
+    rng.flatArray3(r);
     if (al1 > al2 * r[0]) {
       eps = vexp(-al1 * r[1]);
       eps2 = eps * eps;
@@ -1401,7 +1436,7 @@ template <typename R> HD void ConvPerform(const DevTables<R>& T, Trk<R>& t, SecL
       // function: written once, so a wave with lanes in both branches
       // evaluates them once (same operations per lane as the branches)
       do {
-        rng.flatArray(3, r);
+        rng.flatArray3(r);
         const bool first = NormCond > r[0];
         if (first) eps = (R)0.5 - epsRange * cbrt13(r[1]);
         else eps = epsMin + epsRange * r[1];
@@ -1414,7 +1449,7 @@ template <typename R> HD void ConvPerform(const DevTables<R>& T, Trk<R>& t, SecL
     } else {  // SampleEnergyRateWithLPM :203-237
       const R z23 = (R)T.elZ23[z], ilVarS1 = (R)T.elILS1[z], ilVarS1Cond = (R)T.elILS1Cond[z];
       do {
-        rng.flatArray(3, r);
+        rng.flatArray3(r);
         R fXi, fG, fPhi, phi1, phi2;
         if (NormCond > r[0]) {
           eps = (R)0.5 - epsRange * cbrt13(r[1]);
@@ -1510,7 +1545,7 @@ template <typename R> HD void PEPerform(const DevTables<R>& T, Trk<R>& t, R peMx
     const R gtmax = (R)2.0 * (a1 + (R)1.0 / ac);
     R tsam, gtr, r[2];
     do {
-      rng.flatArray(2, r);
+      rng.flatArray2(r);
       tsam = (R)2.0 * ac * ((R)2.0 * r[0] + a2 * dsqrt(r[0])) / (a2 * a2 - (R)4.0 * r[0]);
       gtr = ((R)2.0 - tsam) * (a1 + (R)1.0 / (ac + tsam));
     } while (r[1] * gtmax > gtr);

@@ -47,9 +47,7 @@ template <typename R> HD void LoopBegin(const DevTables<R>& T, ElState<R>& el, S
   L.preEkin = t.ekin;
   L.preLEkin = t.logE();
   L.cont = T.regMultiStep[T.mcReg[t.imc]] != 0;
-#pragma unroll
-  for (int ip = 0; ip < 4; ++ip)
-    if (t.nial[ip] <= (R)0.) t.nial[ip] = -vlog((R)rng.flat());
+  SampleNumIALeft(t.nial, rng);
   HowFarToDiscreteInteraction(T, el);
   L.iDProc = t.winner;
   L.stepLeft = el.pstep;
