@@ -135,6 +135,28 @@ HD uint32_t Xor3(uint32_t a, uint32_t b, uint32_t c) {
 #endif
 }
 
+// a / n, rounded as a division rounds it, for n in [1, kPoissonSmall]: with the
+// nearest double (float) r to 1 / n, q = a * r is within 2 ulp, its remainder
+// a - n q is exact (n has at most 5 bits) and q + r (a - n q) is off by less
+// than 2^-45 ulp, while a / n is either representable or at least 1 / (2 n) ulp
+// from a rounding boundary. (Compared on the host: every float mantissa and
+// 10^8 doubles, half of them next to a multiple of n, without a difference.)
+constexpr int kPoissonSmall = 24;
+__constant__ double kRecip[kPoissonSmall + 1] = {0., 1. / 1., 1. / 2., 1. / 3., 1. / 4., 1. / 5., 1. / 6., 1. / 7., 1. / 8.,
+  1. / 9., 1. / 10., 1. / 11., 1. / 12., 1. / 13., 1. / 14., 1. / 15., 1. / 16., 1. / 17., 1. / 18., 1. / 19., 1. / 20.,
+  1. / 21., 1. / 22., 1. / 23., 1. / 24.};
+__constant__ float kRecipF[kPoissonSmall + 1] = {0.f, 1.f / 1.f, 1.f / 2.f, 1.f / 3.f, 1.f / 4.f, 1.f / 5.f, 1.f / 6.f,
+  1.f / 7.f, 1.f / 8.f, 1.f / 9.f, 1.f / 10.f, 1.f / 11.f, 1.f / 12.f, 1.f / 13.f, 1.f / 14.f, 1.f / 15.f, 1.f / 16.f,
+  1.f / 17.f, 1.f / 18.f, 1.f / 19.f, 1.f / 20.f, 1.f / 21.f, 1.f / 22.f, 1.f / 23.f, 1.f / 24.f};
+HD double DivSmall(double a, int n) {
+  const double r = kRecip[n], q = a * r;
+  return __builtin_fma(__builtin_fma(-(double)n, q, a), r, q);
+}
+HD float DivSmall(float a, int n) {
+  const float r = kRecipF[n], q = a * r;
+  return __builtin_fmaf(__builtin_fmaf(-(float)n, q, a), r, q);
+}
+
 // ---- per-track random stream ------------------------------------------------------------
 // Philox4x32-10 (J. Salmon et al., "Parallel random numbers: as easy as 1, 2, 3",
 // SC'11). Draw d of track `id` comes from block counter {d/2, id, 0, 0}; double j
@@ -276,7 +298,15 @@ struct Rng {
       R poissonSum = poissonValue;
       // kPoissonMaxTerms bounds the summation; for mean <= 16 the sum reaches 1
       // within double rounding long before it, so the bound can only act where
-      // the unbounded loop would never end (a sum saturating below `position`)
+      // the unbounded loop would never end (a sum saturating below `position`).
+      // `number` is the same in every lane of the loop, so mean / number for
+      // small numbers is three instructions on a reciprocal held in scalar
+      // registers (DivSmall) instead of a division's eleven.
+      while (poissonSum <= position && number < kPoissonSmall) {
+        ++number;
+        poissonValue *= DivSmall(mean, number);
+        poissonSum += poissonValue;
+      }
       while (poissonSum <= position && number < kPoissonMaxTerms) {
         ++number;
         poissonValue *= mean / (R)number;
