@@ -1164,7 +1164,7 @@ template <typename R> HD bool SampleLossFluctuations(const DevTables<R>& T, ElSt
   return stopped;
 }
 
-template <typename R> HD bool CheckDelta(const DevTables<R>& T, Trk<R>& t, R rnd) {  // :408-423
+template <typename R> HD bool CheckDelta(const DevTables<R>& T, Trk<R>& t, R winnerMfp, R rnd) {  // :408-423
   const DevEl<R>& e = T.el[t.isEl ? 0 : 1];
   const int iDProc = t.winner;
   const int imc = t.imc;
@@ -1173,7 +1173,7 @@ template <typename R> HD bool CheckDelta(const DevTables<R>& T, Trk<R>& t, R rnd
   const R lekin = t.logE();
   const R mxsec = iDProc < 2 ? GetRestMacXSec(e, imc, ekin, lekin, iDProc == 0)
                 : (iDProc < 3 ? MacXsecAnnihilation((R)ekin, (R)T.matElDens[imat]) : GetMacXSecNuclear(e, imat, ekin, lekin));
-  return mxsec <= (R)0.0 || rnd > mxsec * PickMFP(t.mfp, iDProc);
+  return mxsec <= (R)0.0 || rnd > mxsec * winnerMfp;
 }
 
 // PerformDiscrete (:425-441) up to the final-state sampling: the
@@ -1184,7 +1184,7 @@ template <typename R> HD int ElectronSelectDiscrete(const DevTables<R>& T, Trk<R
   const int iDProc = t.winner;
   if (iDProc < 0 || t.onBoundary) return -1;
   ResetNumIALeft(t.nial, iDProc);
-  if (CheckDelta(T, t, (R)rng.flat())) return -1;
+  if (CheckDelta(T, t, PickMFP(t.mfp, iDProc), (R)rng.flat())) return -1;
   return iDProc;
 }
 
@@ -1233,20 +1233,29 @@ template <typename R> HD void ElectronHowFar(const DevTables<R>& T, ElState<R>& 
 }
 
 // G4HepEmElectronManager::Perform(data, pars, tlData) (:461-483) up to
-// PerformDiscrete: PerformContinuous (:375-405). Returns 1 if the track
-// stopped in the step, 0 if it goes on to PerformDiscrete and -1 for a zero
-// geometrical step (nothing else happens in the step).
-template <typename R> HD int ElectronPerformContinuous(const DevTables<R>& T, ElState<R>& el, Rng& rng) {
+// PerformDiscrete: PerformContinuous (:375-405), in two parts between which the
+// step's length and the interaction lengths left are final and el.t.mfp is
+// needed only for the winner.
+enum ContStep : int { kNoMove = -1, kZeroStep = 0, kMoved = 1 };
+template <typename R> HD ContStep ElectronBeginContinuous(ElState<R>& el) {
   Trk<R>& t = el.t;
   t.edep = 0;
   el.pstep = t.gstep;
-  if (t.gstep <= (R)0.) return -1;
+  if (t.gstep <= (R)0.) return kNoMove;
   el.preEkin = t.ekin;
   el.preLEkin = t.logE();
   UpdatePStepLength(el);
+  if (!(el.pstep > (R)0.0)) return kZeroStep;  // PerformContinuous returns "not stopped" on a zero step
+  UpdateNumIALeft(el);
+  return kMoved;
+}
+// 1 if the track stopped in the step, 0 if it goes on to PerformDiscrete and -1
+// for a zero geometrical step (nothing else happens in the step).
+template <typename R> HD int ElectronPerformContinuous(const DevTables<R>& T, ElState<R>& el, Rng& rng) {
+  const ContStep go = ElectronBeginContinuous(el);
+  if (go == kNoMove) return -1;
   bool stopped = false;
-  if (el.pstep > (R)0.0) {  // PerformContinuous returns "not stopped" on a zero step
-    UpdateNumIALeft(el);
+  if (go == kMoved) {
     stopped = ApplyMeanEnergyLoss(T, el);
     if (!stopped) {
       SampleMSC(T, el, rng);
