@@ -1108,9 +1108,10 @@ __global__ void __launch_bounds__(kBlock, 4) k_step_select_local_batched(DevTabl
   int tile, chunk;
   if (!LocalSelectChunk(ntiles, tile, chunk)) return;
   const int b = __builtin_amdgcn_readfirstlane((int)tbatch[tile]);
-  const hepem_tracks in = d[b].in;
-  hepem_tracks out = d[b].out;
-  const hepem_step_out res = d[b].res;
+  // by reference: copies would keep 84 scalar registers of pointers alive
+  const hepem_tracks& in = d[b].in;
+  hepem_tracks& out = const_cast<hepem_tracks&>(d[b].out);
+  const hepem_step_out& res = d[b].res;
   const int n = in.n;
   const int tile0 = (tile - (int)d[b].tile0) * kClassifyTile;
   const int m = min(kClassifyTile, n - tile0);
@@ -1203,7 +1204,7 @@ __device__ void InteractBatchedTile(const DevTables<R>& T, uint64_t seed, const 
                                     const uint8_t* __restrict__ code, const Staged* __restrict__ st,
                                     const uint16_t* __restrict__ tlist, const uint32_t* __restrict__ tinfo) {
   const int b = __builtin_amdgcn_readfirstlane((int)tbatch[tile]);
-  hepem_tracks out = d[b].out;
+  hepem_tracks& out = const_cast<hepem_tracks&>(d[b].out);
   const uint32_t qoff = d[b].qoff;
   InteractTileChunk<R>(T, seed, out, d[b].res, out.n, code + qoff, st + qoff, tlist + qoff, tinfo + (size_t)tile * kTileInfo,
                        (int)(tile - d[b].ptile0[TI]) * TileSlots(TI), chunk);
