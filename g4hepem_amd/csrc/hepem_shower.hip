@@ -2,15 +2,15 @@
 //
 // The track stack is a pair of structure-of-arrays buffers of `capacity`
 // slots. One stepping round over the n tracks in flight:
-//   k_sh_el_substep  the e-/e+ (the first part of the stack): one sub-step of
+//   k_sh_move      the e-/e+ (the first part of the stack): one sub-step of
 //                  G4HepEmTrackingManager::TrackElectron's step each, after
 //                  the step's pre-step part where a track is not within a step
 //                  (device/dev_tracking.hh), with the slab as the geometry and
 //                  the MSC displacement applied; a track within its step
-//                  carries the loop state to the next round
-//   k_sh_el_end    the e-/e+ whose step ended: the loss fluctuation, at-rest
-//                  annihilation or the discrete interaction
-//   k_sh_gamma     the gammas: HowFar, the cut at the next plane along x (or,
+//                  carries the loop state to the next round, one whose step
+//                  ended finishes it: the loss fluctuation, at-rest
+//                  annihilation or the discrete interaction;
+//                  the gammas: HowFar, the cut at the next plane along x (or,
 //                  with Woodcock tracking on and above its energy limit, a
 //                  step through the stack to its next interaction point or out
 //                  of it), then the boundary update or SelectInteraction +
@@ -94,12 +94,10 @@ __device__ inline int AbsorberCouple(const Slabs& g, int a) {
 // one stack buffer
 // What an e-/e+ carries between the sub-steps of one TrackElectron step
 // (G4HepEmTrackingManager.cc:427-606), which run one per stepping round: the
-// step's pre-step part sets it and each sub-step updates it (k_sh_el_substep),
-// the step's end reads it (k_sh_el_end). Gamma slots do not carry it.
+// step's pre-step part sets it and each sub-step updates it. Gamma slots do not
+// carry it.
 constexpr uint8_t kInStep = 1;   // between sub-steps of a step (else the next round begins a step)
 constexpr uint8_t kCont = 2;     // continueStepping: MSC may limit the next sub-step too
-constexpr uint8_t kStopped = 4;  // the step's last sub-step stopped the track
-constexpr uint8_t kLeft = 8;     // the step's last sub-step left the world
 struct ElLoop {
   double* range;       // restricted range, reduced over the sub-steps
   double* stepLeft;    // what is left of the discrete step
@@ -108,8 +106,7 @@ struct ElLoop {
   double* meanLoss;    // summed mean energy losses
   int32_t* nsub;       // sub-steps taken in the step
   int8_t* iDProc;      // the discrete process HowFarToDiscreteInteraction chose
-  int8_t* winner;      // the process that limited the last sub-step
-  uint8_t* flags;      // kInStep | kCont | kStopped | kLeft
+  uint8_t* flags;      // kInStep | kCont, or 0
 };
 
 struct Stack {
@@ -289,31 +286,25 @@ __device__ bool WoodcockStep(const hepem::DevTables<R>& T, const Slabs& g, hepem
   return true;
 }
 
-// The e-/e+ slots [0, ne) of G4HepEmTrackingManager::TrackElectron's step with
+// Slot i of the e-/e+ part of G4HepEmTrackingManager::TrackElectron's step with
 // the slab as the caller's geometry (device/dev_tracking.hh), one sub-step
-// per stepping round: every slot takes one sub-step, after beginning a step
-// if it is not within one (k_sh_el_substep), and a slot whose step thereby
-// ended finishes it (k_sh_el_end). A slot within a step stays in the stack
-// with its loop state, deposits nothing and creates nothing until its step
-// ends. Every round thus does one uniform unit of work per e-/e+, whatever the
-// length of its sub-step chain.
-//
-// k_sh_el_substep: for a slot not within a step, the pre-step safety (kept in
-// t.safety for the step), the interaction lengths and
-// HowFarToDiscreteInteraction; then one sub-step (SlabSubstep: HowFarToMSC,
-// the move, the along-step part, the MSC displacement). xend = post-sub-step
-// position; side = +1/-1 when it ended on the upper or lower plane of its
-// slab, 0 inside. A slot still within its step gets no deposit or
-// secondaries this round.
+// per stepping round, after beginning a step if the slot is not within one: the
+// pre-step safety (kept in t.safety for the step), the interaction lengths and
+// HowFarToDiscreteInteraction; then SlabSubstep (HowFarToMSC, the move, the
+// along-step part, the MSC displacement). xend = post-sub-step position; side =
+// +1/-1 when it ended on the upper or lower plane of its slab, 0 inside. A slot
+// within a step stays in the stack with its loop state, deposits nothing and
+// creates nothing until its step ends; then the end of the step follows here:
+// the loss fluctuation on the summed mean loss, at-rest annihilation, or the
+// choice of the discrete interaction and its final state. Every round thus does
+// one uniform unit of work per e-/e+, whatever the length of its sub-step chain.
 template <typename R>
-__global__ void __launch_bounds__(kB) k_sh_el_substep(Stack s, Slabs g, hepem_step_out res, double* __restrict__ xend,
-                                                      int8_t* __restrict__ side, hepem::DevTables<R> T, uint64_t seed,
-                                                      int ne) {
+__device__ __forceinline__ void ElectronSubstep(const Stack& s, const Slabs& g, const hepem_step_out& res,
+                                                double* __restrict__ xend, int8_t* __restrict__ side,
+                                                const hepem::DevTables<R>& T, uint64_t seed, int i) {
   using namespace hepem;
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= ne) return;
   const int n = s.t.n;
-  hepem_tracks& t = s.t;
+  hepem_tracks t = s.t;
   const int l = s.layer[i];
   ElState<R> el;
   Rng rng;
@@ -349,81 +340,56 @@ __global__ void __launch_bounds__(kB) k_sh_el_substep(Stack s, Slabs g, hepem_st
     L.nsub = s.lp.nsub[i];
   }
   const bool done = SlabSubstep(T, el, L, rng, p);
-  StoreElectronState(t, n, i, el, rng);
-  t.ekin[i] = el.t.ekin;
-#pragma unroll
-  for (int c = 0; c < 3; ++c) t.dir[c * n + i] = (double)el.t.dir[c];
+  const R rangeLeft = el.range;
   t.on_boundary[i] = p.side != 0 ? 1 : 0;
-  s.lp.range[i] = (double)el.range;
-  s.lp.stepLeft[i] = (double)L.stepLeft;
-  s.lp.meanLoss[i] = L.meanLoss;
-  s.lp.nsub[i] = L.nsub;
-  s.lp.winner[i] = (int8_t)el.t.winner;
-  s.lp.flags[i] = done ? (uint8_t)((L.stopped ? kStopped : 0) | (L.left ? kLeft : 0)) : (uint8_t)(kInStep | kCont);
-  if (!done) {
-    res.edep[i] = 0.0;
-    res.nsec[i] = 0;
-  }
   xend[i] = p.x;
   side[i] = (int8_t)p.side;
-}
-
-// k_sh_el_end: the step's end for the slots whose step ended this round: the
-// loss fluctuation on the summed mean loss, at-rest annihilation, or the choice
-// of the discrete interaction and its final state (LoopFinish).
-template <typename R>
-__global__ void __launch_bounds__(kB) k_sh_el_end(Stack s, hepem_step_out res, hepem::DevTables<R> T, uint64_t seed, int ne) {
-  using namespace hepem;
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= ne) return;
-  const uint8_t f = s.lp.flags[i];
-  if (f & kInStep) return;
-  const int n = s.t.n;
-  hepem_tracks& t = s.t;
-  ElState<R> el;
-  Rng rng;
-  InitElectron(t, n, i, seed, el, rng);
-#pragma unroll
-  for (int k = 0; k < 4; ++k) el.t.mfp[k] = (R)s.lp.mfp[k * n + i];
-  el.range = (R)s.lp.range[i];
-  el.t.winner = s.lp.winner[i];
-  StepLoop<R> L;
-  L.iDProc = s.lp.iDProc[i];
-  L.meanLoss = s.lp.meanLoss[i];
-  L.preEkin = s.lp.preEkin[i];
-  L.preLEkin = L.preEkin > 0. ? vlog((R)L.preEkin) : (R)-30;
-  L.stopped = (f & kStopped) != 0;
-  L.left = (f & kLeft) != 0;
-  L.cont = false;
+  {
+    const Msc<R>& m = el.msc;
+    t.msc_init_range[i] = (double)m.initRange;
+    t.msc_dyn_range_factor[i] = (double)m.dynRangeFactor;
+    t.msc_tlimit_min[i] = (double)m.tlimitMin;
+    t.msc_first_step[i] = m.firstStep ? 1 : 0;
+  }
   SecList<R> sl;
   sl.ns = 0;
-  const int p = LoopFinishSelect(T, el, L, sl, rng);
-  res.edep[i] = el.t.edep;
-  res.winner[i] = el.t.winner;
-  ElectronFinalState(T, el.t, p, sl, rng);
+  double edep = 0.0;
+  if (done) {
+    L.preLEkin = L.preEkin > 0. ? vlog((R)L.preEkin) : (R)-30;
+    s.lp.flags[i] = 0;
+    const int proc = LoopFinishSelect(T, el, L, sl, rng);
+    edep = el.t.edep;
+    ElectronFinalState(T, el.t, proc, sl, rng);
+  } else {
+    s.lp.range[i] = (double)rangeLeft;
+    s.lp.stepLeft[i] = (double)L.stepLeft;
+    s.lp.meanLoss[i] = L.meanLoss;
+    s.lp.nsub[i] = L.nsub;
+    s.lp.flags[i] = (uint8_t)(kInStep | kCont);
+  }
+  res.edep[i] = edep;
+#pragma unroll
+  for (int k = 0; k < 4; ++k) t.num_ia_left[k * n + i] = (double)el.t.nial[k];
   t.ekin[i] = el.t.ekin;
 #pragma unroll
   for (int c = 0; c < 3; ++c) t.dir[c * n + i] = (double)el.t.dir[c];
-#pragma unroll
-  for (int k = 0; k < 4; ++k) t.num_ia_left[k * n + i] = (double)el.t.nial[k];
   StoreRng(t, i, rng);
   WriteSecondaries(res, n, i, sl);
 }
 
-// One step of the gamma slots [ne, n), as G4HepEmTrackingManager::TrackGamma
+// One step of gamma slot i, as G4HepEmTrackingManager::TrackGamma
 // takes it (G4HepEmTrackingManager.cc:893-1145): HowFar, the cut at the next
 // plane along x (or, with Woodcock tracking on and above its energy limit, a
 // Woodcock step through the stack), then the boundary update or
-// SelectInteraction + Perform. xend and side as k_sh_el_substep; layer = the slab
+// SelectInteraction + Perform. xend and side as ElectronSubstep; layer = the slab
 // the step's deposit is scored in (changed only by a Woodcock step).
 template <typename R, bool kWoodcock>
-__global__ void __launch_bounds__(kB) k_sh_gamma(Stack s, Slabs g, hepem_step_out res, double* __restrict__ xend,
-                                                 int8_t* __restrict__ side, hepem::DevTables<R> T, uint64_t seed, int ne) {
+__device__ __forceinline__ void GammaStep(const Stack& s, const Slabs& g, const hepem_step_out& res,
+                                          double* __restrict__ xend, int8_t* __restrict__ side,
+                                          const hepem::DevTables<R>& T, uint64_t seed, int i) {
   using namespace hepem;
-  const int i = ne + blockIdx.x * blockDim.x + threadIdx.x;
   const int n = s.t.n;
-  if (i >= n) return;
-  hepem_tracks& t = s.t;
+  hepem_tracks t = s.t;
   int l = s.layer[i];
   const double x = s.x[i];
   SecList<R> sl;
@@ -467,12 +433,31 @@ __global__ void __launch_bounds__(kB) k_sh_gamma(Stack s, Slabs g, hepem_step_ou
   t.num_ia_left[i] = (double)gt.nial[0];
   StoreRng(t, i, rng);
   t.on_boundary[i] = gt.onBoundary ? 1 : 0;
-  res.true_step[i] = (double)gt.gstep;
   res.edep[i] = gt.edep;
-  res.winner[i] = gt.winner;
   WriteSecondaries(res, n, i, sl);
   xend[i] = xe;
   side[i] = (int8_t)sd;
+}
+
+// One sub-step of the e-/e+ slots [0, ne) in the first `ge` blocks and one step
+// of the gamma slots [ne, n) in the others. Bound by the latency of one wave's
+// chain as long as a round leaves most SIMDs with a wave or two of each kind:
+// in one launch the gamma waves run beside the e-/e+ waves instead of after
+// them, and an e-/e+ whose step ends goes on with its state in registers. Per
+// round of 1000 showers 73 us, against 38 for the sub-steps, 36 for the steps'
+// ends and 32 for the gammas in kernels of their own. Held to the waves per
+// SIMD that those kernels had (3 in FP64, 4 in the FP32-table form).
+template <typename R, bool kWoodcock>
+__global__ void __launch_bounds__(kB, sizeof(R) == sizeof(double) ? 3 : 4) k_sh_move(Stack s, Slabs g, hepem_step_out res, double* __restrict__ xend,
+                                                int8_t* __restrict__ side, hepem::DevTables<R> T, uint64_t seed, int ne,
+                                                int ge) {
+  if ((int)blockIdx.x < ge) {
+    const int i = (int)blockIdx.x * kB + (int)threadIdx.x;
+    if (i < ne) ElectronSubstep(s, g, res, xend, side, T, seed, i);
+  } else {
+    const int i = ne + ((int)blockIdx.x - ge) * kB + (int)threadIdx.x;
+    if (i < s.t.n) GammaStep<R, kWoodcock>(s, g, res, xend, side, T, seed, i);
+  }
 }
 
 // After Perform: position, slab crossing, scoring and next-round slot counts.
@@ -863,7 +848,6 @@ void AskStack(Arena& A, Stack& s, size_t cap) {
   A.get(s.lp.meanLoss, cap);
   A.get(s.lp.nsub, cap);
   A.get(s.lp.iDProc, cap);
-  A.get(s.lp.winner, cap);
   A.get(s.lp.flags, cap);
 }
 
@@ -910,7 +894,9 @@ extern "C" int hepem_slab_run(const hepem_ctx* ctx, const hepem_slab_setup* su, 
   Arena A;
   Stack s[2];
   hepem_step_out res;  // the fields the stepping kernel writes and the post kernel reads
+  res.true_step = nullptr;
   res.geom_step = nullptr;
+  res.winner = nullptr;
   res.displacement = nullptr;
   res.stopped = nullptr;
   double *dPlanes, *xend;
@@ -921,9 +907,7 @@ extern "C" int hepem_slab_run(const hepem_ctx* ctx, const hepem_slab_setup* su, 
   const int nblk = (cap + kB - 1) / kB;
   AskStack(A, s[0], (size_t)cap);
   AskStack(A, s[1], (size_t)cap);
-  A.get(res.true_step, (size_t)cap);
   A.get(res.edep, (size_t)cap);
-  A.get(res.winner, (size_t)cap);
   A.get(res.nsec, (size_t)cap);
   A.get(res.sec_ptype, 2 * (size_t)cap);
   A.get(res.sec_ekin, 2 * (size_t)cap);
@@ -1038,28 +1022,15 @@ extern "C" int hepem_slab_run(const hepem_ctx* ctx, const hepem_slab_setup* su, 
       const int grid = (n + kB - 1) / kB;
       // the e-/e+ part of the stack comes first
       const int ge = (ne + kB - 1) / kB, gg = (n - ne + kB - 1) / kB;
-      if (ge > 0) {
-        if (fp64) {
-          hipLaunchKernelGGL(k_sh_el_substep<double>, dim3(ge), dim3(kB), 0, st, a, g, res, xend, side, HepemTables64(ctx),
-                             seed, ne);
-          hipLaunchKernelGGL(k_sh_el_end<double>, dim3(ge), dim3(kB), 0, st, a, res, HepemTables64(ctx), seed, ne);
-        } else {
-          hipLaunchKernelGGL(k_sh_el_substep<float>, dim3(ge), dim3(kB), 0, st, a, g, res, xend, side, HepemTables32(ctx),
-                             seed, ne);
-          hipLaunchKernelGGL(k_sh_el_end<float>, dim3(ge), dim3(kB), 0, st, a, res, HepemTables32(ctx), seed, ne);
-        }
-        r->substeps += ne;
-      }
-      if (gg > 0) {
-        if (fp64 && woodcock)
-          hipLaunchKernelGGL((k_sh_gamma<double, true>), dim3(gg), dim3(kB), 0, st, a, g, res, xend, side, HepemTables64(ctx), seed, ne);
-        else if (fp64)
-          hipLaunchKernelGGL((k_sh_gamma<double, false>), dim3(gg), dim3(kB), 0, st, a, g, res, xend, side, HepemTables64(ctx), seed, ne);
-        else if (woodcock)
-          hipLaunchKernelGGL((k_sh_gamma<float, true>), dim3(gg), dim3(kB), 0, st, a, g, res, xend, side, HepemTables32(ctx), seed, ne);
-        else
-          hipLaunchKernelGGL((k_sh_gamma<float, false>), dim3(gg), dim3(kB), 0, st, a, g, res, xend, side, HepemTables32(ctx), seed, ne);
-      }
+      if (fp64 && woodcock)
+        hipLaunchKernelGGL((k_sh_move<double, true>), dim3(ge + gg), dim3(kB), 0, st, a, g, res, xend, side, HepemTables64(ctx), seed, ne, ge);
+      else if (fp64)
+        hipLaunchKernelGGL((k_sh_move<double, false>), dim3(ge + gg), dim3(kB), 0, st, a, g, res, xend, side, HepemTables64(ctx), seed, ne, ge);
+      else if (woodcock)
+        hipLaunchKernelGGL((k_sh_move<float, true>), dim3(ge + gg), dim3(kB), 0, st, a, g, res, xend, side, HepemTables32(ctx), seed, ne, ge);
+      else
+        hipLaunchKernelGGL((k_sh_move<float, false>), dim3(ge + gg), dim3(kB), 0, st, a, g, res, xend, side, HepemTables32(ctx), seed, ne, ge);
+      r->substeps += ne;
       hipLaunchKernelGGL(k_sh_post, dim3(grid), dim3(kB), 0, st, a, g, res, xend, side, dep, leak, keep, smask, offs, offs + cap,
                          bsum, bsum + nblk, bsec);
       // primaries of the next events join once the stack runs low, and no
