@@ -362,6 +362,10 @@ HD uint8_t ElectronSelectAfterHowFar(const DevTables<R>& T, ElState<R>& el, Rng&
 #pragma unroll
   for (int k = 0; k < 4; ++k)
     if (k != winner) out.num_ia_left[k * n + i] = (double)t.nial[k];
+  // the direction is not needed before the scattering turns it: loaded here, it
+  // holds no registers through HowFar
+#pragma unroll
+  for (int c = 0; c < 3; ++c) t.dir[c] = (R)in.dir[c * n + i];
   bool stopped = false;
   if (go == kMoved) {
     stopped = ApplyMeanEnergyLoss(T, el);
@@ -395,18 +399,6 @@ HD uint8_t ElectronSelectAfterHowFar(const DevTables<R>& T, ElState<R>& el, Rng&
   res.stopped[i] = t.ekin <= 0.0 ? 1 : 0;
   WriteSecondaries(res, n, i, sl);
   return kPNone;
-}
-
-// Stage 1 of an e-/e+ slot of the fused step: as StepElectron up to
-// PerformDiscrete's choice.
-template <typename R>
-HD uint8_t StepElectronSelect(const DevTables<R>& T, uint64_t seed, const hepem_tracks& in, hepem_tracks& out,
-                              const hepem_step_out& res, Staged* st, int n, int i) {
-  ElState<R> el;
-  Rng rng;
-  InitElectron(in, n, i, seed, el, rng);
-  ElectronHowFar(T, el, rng);
-  return ElectronSelectAfterHowFar(T, el, rng, in, out, res, st, n, i);
 }
 
 // Stage 1 of an e-/e+ slot of the split Perform: the HowFar state comes from
@@ -461,17 +453,37 @@ HD uint8_t GammaSelectAfterHowFar(const DevTables<R>& T, Trk<R>& t, R pe, Rng& r
   return kPNone;
 }
 
-// Stage 1 of a gamma slot of the fused step: HowFar, then as above.
+// Stage 1 of slot i of the step: its whole state loaded at once, the test of
+// its couple and energy, the identity copy, HowFar and the selection. Records
+// the slot's code.
 template <typename R>
-HD uint8_t StepGammaSelect(const DevTables<R>& T, uint64_t seed, const hepem_tracks& in, hepem_tracks& out,
-                           const hepem_step_out& res, Staged* st, int n, int i) {
-  Trk<R> t;
-  t.isEl = false;
-  LoadTrack(in, n, i, t);
+HD void StepSelect(const DevTables<R>& T, uint64_t seed, const hepem_tracks& in, hepem_tracks& out, const hepem_step_out& res,
+                   uint32_t* counters, uint8_t* code, Staged* st, int n, int i, bool isE) {
+  TrackIn r = LoadTrackIn(in, n, i);
+  MscIn q{};
+  if (isE) q = LoadMscIn(in, i);
+  KeepLoaded(r);
+  if (!TrackValid(T, r.imc, r.ekin)) {
+    atomicAdd(&counters[2], 1u);
+    WriteRejected<R>(in, out, res, n, i);
+    code[i] = kPNone;
+    return;
+  }
+  StoreIdentity(in, out, i, r);
   Rng rng;
-  rng.init(seed, (uint32_t)in.id[i], StreamHi(in, i), in.rng_ctr[i], in.rng_has_gauss[i] != 0, in.rng_gauss[i]);
-  const R pe = GammaHowFar(T, t, rng);
-  return GammaSelectAfterHowFar(T, t, pe, rng, in, out, res, st, n, i);
+  if (isE) {
+    ElState<R> el;
+    InitElectron(r, q, seed, el, rng);
+    ElectronHowFar(T, el, rng);
+    code[i] = ElectronSelectAfterHowFar(T, el, rng, in, out, res, st, n, i);
+  } else {
+    Trk<R> t;
+    t.isEl = false;
+    InitTrack(r, t);
+    InitRng(r, seed, rng);
+    const R pe = GammaHowFar(T, t, rng);
+    code[i] = GammaSelectAfterHowFar(T, t, pe, rng, in, out, res, st, n, i);
+  }
 }
 
 // Stage 1 of a gamma slot of the split Perform: step, mean free path and PE
@@ -699,12 +711,7 @@ __global__ void __launch_bounds__(kBlock, 4) k_step_select_local(DevTables<R> T,
   // the layout hepem_step_prepare chose: tile-local, or e-/e+ first over the batch
   const bool isE = counters[kCounterLayout] ? jl < (int)tinfo[(size_t)tile * kTileInfo] : (uint32_t)(tile0 + jl) < counters[0];
   const int i = (int)queue[tile0 + jl];
-  if (RejectTrack(T, in, out, res, n, i, counters)) {
-    code[i] = kPNone;
-    return;
-  }
-  CopyIdentity(in, out, i);
-  code[i] = isE ? StepElectronSelect(T, seed, in, out, res, st, n, i) : StepGammaSelect(T, seed, in, out, res, st, n, i);
+  StepSelect(T, seed, in, out, res, counters, code, st, n, i, isE);
 }
 
 // Thread -> (slot, is-e-/e+) of the split HowFar and Perform kernels. A
@@ -961,12 +968,27 @@ __device__ void InteractTileChunk(const DevTables<R>& T, uint64_t seed, hepem_tr
                                   const uint8_t* __restrict__ code, const Staged* __restrict__ st,
                                   const uint16_t* __restrict__ tlist, const uint32_t* __restrict__ info, int tile0,
                                   uint32_t chunk) {
-  if (chunk >= info[2 * kNumProc + 1]) return;
+  // the chunk is the same for the whole wave: its process is found in scalar
+  // registers from one load of the tile's words (a search through them in
+  // memory was a chain of up to eight dependent loads)
+  chunk = (uint32_t)__builtin_amdgcn_readfirstlane((int)chunk);
+  uint32_t w[kTileInfo];
+#pragma unroll
+  for (int k = 0; k < kTileInfo; ++k) w[k] = info[k];
+  if (chunk >= w[2 * kNumProc + 1]) return;
   int q = 0;
-  while (q + 1 < kNumProc && chunk >= info[kNumProc + 2 + q]) ++q;
-  const uint32_t k = (chunk - info[kNumProc + 1 + q]) * 64u + (uint32_t)__lane_id();
-  if (k >= info[q + 1] - info[q]) return;
-  const int i = tile0 + (int)tlist[tile0 + info[q] + k];
+  uint32_t first = w[0], end = w[1], chunk0 = w[kNumProc + 1];
+#pragma unroll
+  for (int p = 1; p < kNumProc; ++p) {
+    const bool here = chunk >= w[kNumProc + 1 + p];
+    q = here ? p : q;
+    first = here ? w[p] : first;
+    end = here ? w[p + 1] : end;
+    chunk0 = here ? w[kNumProc + 1 + p] : chunk0;
+  }
+  const uint32_t k = (chunk - chunk0) * 64u + (uint32_t)__lane_id();
+  if (k >= end - first) return;
+  const int i = tile0 + (int)tlist[tile0 + first + k];
   const uint8_t c = code[i];
   const Staged r = st[i];
   if (q + 1 < kPConv) ElectronInteract<R>(T, seed, out, res, n, i, r, c);
@@ -1071,14 +1093,7 @@ __device__ void StepSelectChunk(const DevTables<R>& T, uint64_t seed, const Batc
   uint32_t* cnt = bcounters + 4 * b;
   const uint32_t qoff = d[b].qoff;
   const int i = (int)queue[qoff + j];
-  uint8_t* cb = code + qoff;
-  if (RejectTrack(T, in, out, res, n, i, cnt)) {
-    cb[i] = kPNone;
-    return;
-  }
-  CopyIdentity(in, out, i);
-  cb[i] = (uint32_t)j < cnt[0] ? StepElectronSelect(T, seed, in, out, res, st + qoff, n, i)
-                               : StepGammaSelect(T, seed, in, out, res, st + qoff, n, i);
+  StepSelect(T, seed, in, out, res, cnt, code + qoff, st + qoff, n, i, (uint32_t)j < cnt[0]);
 }
 
 // The tile-local particle partition over every batch: block t lays out
@@ -1119,14 +1134,7 @@ __global__ void __launch_bounds__(kBlock, 4) k_step_select_local_batched(DevTabl
   if (jl >= m) return;
   const uint32_t qoff = d[b].qoff;
   const int i = (int)queue[qoff + tile0 + jl];
-  uint8_t* cb = code + qoff;
-  if (RejectTrack(T, in, out, res, n, i, bcounters + 4 * b)) {
-    cb[i] = kPNone;
-    return;
-  }
-  CopyIdentity(in, out, i);
-  cb[i] = jl < (int)ecount[tile] ? StepElectronSelect(T, seed, in, out, res, st + qoff, n, i)
-                                 : StepGammaSelect(T, seed, in, out, res, st + qoff, n, i);
+  StepSelect(T, seed, in, out, res, bcounters + 4 * b, code + qoff, st + qoff, n, i, jl < (int)ecount[tile]);
 }
 
 // Next work item of a persistent kernel: thread 0 takes it from *next and the
