@@ -29,6 +29,23 @@ constexpr int kSBGuide = 32;           // buckets of the SB search guide
 template <typename T> HD T tmax(T a, T b) { return a > b ? a : b; }
 template <typename T> HD T tmin(T a, T b) { return a < b ? a : b; }
 
+// a / b, rounded as a division rounds it, for b and a / b well inside the range
+// of normal numbers (a may be 0): a reciprocal refined twice and a quotient
+// corrected by its exact remainder. A general division also scales its
+// operands and mends special values, three of its eleven instructions, which
+// never act there.
+HD double DivInRange(double a, double b) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  double y = __builtin_amdgcn_rcp(b);
+  y = __builtin_fma(y, __builtin_fma(-b, y, 1.0), y);
+  y = __builtin_fma(y, __builtin_fma(-b, y, 1.0), y);
+  const double q = a * y;
+  return __builtin_fma(__builtin_fma(-b, q, a), y, q);
+#else
+  return a / b;
+#endif
+}
+
 // ---- exp / log --------------------------------------------------------------------------
 // FP64: the Cephes rational forms (S. L. Moshier's Cephes library, as packaged
 // in VDT and used on the reference host path, G4HepEmExp.hh / G4HepEmLog.hh),
@@ -56,7 +73,7 @@ HD double vexp(double initial_x) {
   qx += 2.27265548208155028766E-1;
   qx *= xx;
   qx += 2.00000000000000000009E0;
-  x = px / (qx - px);
+  x = DivInRange(px, qx - px);  // |x| <= 0.35: the divisor is about 2
   x = 1.0 + 2.0 * x;
   x *= __longlong_as_double((long long)((((uint64_t)(int64_t)n) + 1023) << 52));
   if (initial_x > 708.0) x = __longlong_as_double(0x7FF0000000000000LL);
@@ -89,7 +106,7 @@ HD double vlog(double x) {
   qx *= x; qx += 8.29875266912776603211E1;
   qx *= x; qx += 7.11544750618563894466E1;
   qx *= x; qx += 2.31251620126765340583E1;
-  double res = px / qx;
+  double res = DivInRange(px, qx);  // -0.3 < x < 0.42: the divisor lies in 8 ... 71
   res -= fe * 2.121944400546905827679e-4;
   res -= 0.5 * x2;
   res = x + res;
