@@ -14,6 +14,7 @@
 // order and are bit-identical to an unsorted pass.
 #pragma once
 
+#include "device/dev_final.hh"
 #include "device/dev_physics.hh"
 #include "device/dev_soa.hh"
 #include "device/dev_tracking.hh"
@@ -287,47 +288,6 @@ __global__ void __launch_bounds__(kBlock) k_el_end(DevTables<R> T, uint64_t seed
 // sampler. (The batched step does the same over the tiles of all its batches,
 // k_classify_tiles_batched and k_interact_tiles_batched.)
 
-// processes of the second stage (0: none pending), in the low 4 bits of the
-// per-slot code; bit 4: the track is an e-, bit 5: a Gaussian deviate is cached
-enum ProcCode : uint8_t {
-  kPNone = 0,
-  kPIoniEl,    // Moller
-  kPIoniPos,   // Bhabha
-  kPBremSB,    // Seltzer-Berger brem (E < model limit)
-  kPBremRB,    // relativistic brem
-  kPAnnih,     // e+ annihilation in flight
-  kPConv,      // gamma conversion
-  kPCompton,   // Klein-Nishina
-  kPPE,        // photoelectric
-};
-constexpr int kNumProc = 8;          // codes 1..8
-constexpr uint8_t kCodeProc = 0x0F, kCodeElectron = 0x10, kCodeGauss = 0x20;
-
-// state handed from the selection to the final-state sampling of one slot
-struct alignas(16) Staged {
-  double ekin, dir[3], gauss, pe;
-  int32_t imc, id;
-  uint32_t stream, ctr;
-};
-static_assert(sizeof(Staged) == 64, "one 64-byte record per pending slot");
-
-HD uint8_t StageTrack(Staged* st, int i, uint8_t proc, bool isEl, int imc, int32_t id, uint32_t stream, double ekin,
-                      const double* dir, const Rng& rng, double pe) {
-  Staged r;
-  r.ekin = ekin;
-  r.dir[0] = dir[0];
-  r.dir[1] = dir[1];
-  r.dir[2] = dir[2];
-  r.gauss = rng.gauss;
-  r.pe = pe;
-  r.imc = imc;
-  r.id = id;
-  r.stream = stream;
-  r.ctr = rng.ctr;
-  st[i] = r;
-  return (uint8_t)(proc | (isEl ? kCodeElectron : 0) | (rng.has_gauss ? kCodeGauss : 0));
-}
-
 // Stage 1 of an e-/e+ slot after its HowFar: the continuous step and
 // PerformDiscrete's choice (G4HepEmElectronManager.icc:425-441,461-483).
 // Returns the slot code; a complete step (kPNone) also gets its post-step
@@ -383,10 +343,7 @@ HD uint8_t ElectronSelectAfterHowFar(const DevTables<R>& T, ElState<R>& el, Rng&
   if (stopped) {
     if (!t.isEl) AnnihilateAtRest(sl, rng);
   } else if (discrete && !CheckDelta(T, t, winnerMfp, (R)rng.flat())) {
-    proc = winner == 0   ? (t.isEl ? kPIoniEl : kPIoniPos)
-           : winner == 1 ? (t.ekin < T.bremModelLim ? kPBremSB : kPBremRB)
-           : winner == 2 ? kPAnnih
-                         : kPNone;  // e-/e+ nuclear (no final state)
+    proc = ElectronProc(T, t, winner);
   }
   if (proc != kPNone) {
     const double d[3] = {(double)t.dir[0], (double)t.dir[1], (double)t.dir[2]};
@@ -419,17 +376,7 @@ HD uint8_t PerformElectronSelect(const DevTables<R>& T, uint64_t seed, hepem_tra
 template <typename R>
 HD uint8_t GammaSelectAfterHowFar(const DevTables<R>& T, Trk<R>& t, R pe, Rng& rng, const hepem_tracks& in,
                                   hepem_tracks& out, const hepem_step_out& res, Staged* st, int n, int i) {
-  uint8_t proc = kPNone;
-  if (t.onBoundary) {
-    t.nial[0] -= t.gstep / t.mfp[0];
-  } else {
-    SampleInteraction(T, t, pe, (R)rng.flat());
-    if (t.winner != 3) {
-      t.nial[0] -= t.gstep / t.mfp[0];
-      ResetNumIALeft(t.nial, t.winner);
-      proc = t.winner == 0 ? kPConv : t.winner == 1 ? kPCompton : kPPE;
-    }
-  }
+  const uint8_t proc = GammaProc(T, t, pe, rng);
 #pragma unroll
   for (int k = 0; k < 4; ++k) out.num_ia_left[k * n + i] = (double)t.nial[k];
   res.true_step[i] = (double)t.gstep;
@@ -501,17 +448,6 @@ HD uint8_t PerformGammaSelect(const DevTables<R>& T, uint64_t seed, hepem_tracks
   return GammaSelectAfterHowFar(T, g, (R)hs.pe_xsec[i], rng, t, t, res, st, n, i);
 }
 
-// Stage 2: track state of a pending slot from its staged record.
-template <typename R> HD void Unstage(const Staged& r, uint8_t code, uint64_t seed, Trk<R>& t, Rng& rng) {
-  t.isEl = (code & kCodeElectron) != 0;
-  t.setE(r.ekin);
-#pragma unroll
-  for (int c = 0; c < 3; ++c) t.dir[c] = (R)r.dir[c];
-  t.imc = r.imc;
-  t.edep = 0.0;
-  rng.init(seed, (uint32_t)r.id, r.stream, r.ctr, (code & kCodeGauss) != 0, r.gauss);
-}
-
 // Stage 2 of an e-/e+ slot: the final state of the chosen interaction
 // (PerformDiscrete, G4HepEmElectronManager.icc:443-458).
 template <typename R>
@@ -522,13 +458,7 @@ HD void ElectronInteract(const DevTables<R>& T, uint64_t seed, hepem_tracks& out
   Unstage(r, code, seed, t, rng);
   SecList<R> sl;
   sl.ns = 0;
-  switch (code & kCodeProc) {
-    case kPIoniEl:
-    case kPIoniPos: IoniPerform(T, t, sl, rng); break;
-    case kPBremSB: BremPerform(T, t, sl, rng, true); break;
-    case kPBremRB: BremPerform(T, t, sl, rng, false); break;
-    default: AnnihilateInFlight(t, sl, rng); break;
-  }
+  ElectronFinal(T, t, code & kCodeProc, sl, rng);
   out.ekin[i] = t.ekin;
 #pragma unroll
   for (int c = 0; c < 3; ++c) out.dir[c * n + i] = (double)t.dir[c];
@@ -547,16 +477,7 @@ HD void GammaInteract(const DevTables<R>& T, uint64_t seed, hepem_tracks& out, c
   Unstage(r, code, seed, t, rng);
   SecList<R> sl;
   sl.ns = 0;
-  switch (code & kCodeProc) {
-    case kPConv: ConvPerform(T, t, sl, rng); break;
-    case kPCompton: ComptonPerform(t, sl, rng); break;
-    default: PEPerform(T, t, (R)r.pe, sl, rng); break;
-  }
-  const double finalEkin = t.ekin;
-  if (finalEkin > 0.0 && finalEkin <= T.gamTrackCut) {
-    t.setE(0.0);
-    t.edep += finalEkin;
-  }
+  GammaFinal(T, t, code & kCodeProc, (R)r.pe, sl, rng);
   out.ekin[i] = t.ekin;
 #pragma unroll
   for (int c = 0; c < 3; ++c) out.dir[c * n + i] = (double)t.dir[c];

@@ -14,10 +14,10 @@
 //                  with Woodcock tracking on and above its energy limit, a
 //                  step through the stack to its next interaction point or out
 //                  of it), then the boundary update or SelectInteraction +
-//                  Perform
-//   k_sh_post      slab crossing, leakage, scoring, the number of stack slots
-//                  each track needs next round and their exclusive scan within
-//                  the block
+//                  Perform;
+//                  then, for both, slab crossing, leakage, scoring, the stack
+//                  slots each track needs next round and their exclusive scan
+//                  within the block
 //   k_scan_sums    exclusive scans of the block totals (one block)
 //   k_sh_scatter   survivors and their secondaries into the other buffer:
 //                  e-/e+ first, then gammas, each in slot order of the parents
@@ -33,6 +33,7 @@
 #include <new>
 #include <vector>
 
+#include "device/dev_final.hh"
 #include "device/dev_physics.hh"
 #include "device/dev_scan.hh"
 #include "device/dev_soa.hh"
@@ -286,29 +287,65 @@ __device__ bool WoodcockStep(const hepem::DevTables<R>& T, const Slabs& g, hepem
   return true;
 }
 
+// What a slot's step leaves after its final state: kinematics, random stream and
+// secondaries for the scatter, and in place of the slot's staged record what the
+// end of the round needs of it (its energy, the deposit, the secondaries' number,
+// kinds and energies).
+template <typename R>
+__device__ __forceinline__ void StoreFinal(hepem_tracks& t, const hepem_step_out& res, int n, int i, const hepem::Trk<R>& k,
+                                           const hepem::Rng& rng, const hepem::SecList<R>& sl, double edep, hepem::Staged& r) {
+  t.ekin[i] = k.ekin;
+#pragma unroll
+  for (int c = 0; c < 3; ++c) t.dir[c * n + i] = (double)k.dir[c];
+  hepem::StoreRng(t, i, rng);
+  r.ekin = k.ekin;
+  r.dir[0] = edep;
+  r.imc = sl.ns;
+  if (sl.ns > 0) {
+    hepem::WriteSlot<R>(res, n, i, 0, sl.s0);
+    r.dir[1] = sl.s0.ekin;
+    r.id = sl.s0.ptype;
+  }
+  if (sl.ns > 1) {
+    hepem::WriteSlot<R>(res, n, i, 1, sl.s1);
+    r.dir[2] = sl.s1.ekin;
+    r.stream = (uint32_t)sl.s1.ptype;
+  }
+}
+// Where a slot's move ended, held by its thread to the end of the round.
+struct Moved {
+  double x;      // position
+  int layer;     // the slab the deposit is scored in
+  int side;      // +1/-1: on the upper/lower plane of the slab, 0: inside
+  bool ended;    // the step ended (an e-/e+ within its sub-steps has not)
+};
+
 // Slot i of the e-/e+ part of G4HepEmTrackingManager::TrackElectron's step with
 // the slab as the caller's geometry (device/dev_tracking.hh), one sub-step
 // per stepping round, after beginning a step if the slot is not within one: the
 // pre-step safety (kept in t.safety for the step), the interaction lengths and
 // HowFarToDiscreteInteraction; then SlabSubstep (HowFarToMSC, the move, the
-// along-step part, the MSC displacement). xend = post-sub-step position; side =
-// +1/-1 when it ended on the upper or lower plane of its slab, 0 inside. A slot
-// within a step stays in the stack with its loop state, deposits nothing and
+// along-step part, the MSC displacement). A slot within a step stays in the stack with its loop state, deposits nothing and
 // creates nothing until its step ends; then the end of the step follows here:
 // the loss fluctuation on the summed mean loss, at-rest annihilation, or the
-// choice of the discrete interaction and its final state. Every round thus does
-// one uniform unit of work per e-/e+, whatever the length of its sub-step chain.
+// choice of the discrete interaction. Every round thus does one uniform unit of
+// work per e-/e+, whatever the length of its sub-step chain. Returns the code of
+// an interaction whose final state is pending, with its record at st[j] (and the
+// step's deposit in its pe), or 0.
 template <typename R>
-__device__ __forceinline__ void ElectronSubstep(const Stack& s, const Slabs& g, const hepem_step_out& res,
-                                                double* __restrict__ xend, int8_t* __restrict__ side,
-                                                const hepem::DevTables<R>& T, uint64_t seed, int i) {
+__device__ __forceinline__ uint8_t ElectronSubstep(const Stack& s, const Slabs& g, const hepem_step_out& res,
+                                                   const hepem::DevTables<R>& T, uint64_t seed, int i, Moved& mv,
+                                                   hepem::Staged* st, int j) {
   using namespace hepem;
   const int n = s.t.n;
   hepem_tracks t = s.t;
   const int l = s.layer[i];
   ElState<R> el;
   Rng rng;
-  InitElectron(t, n, i, seed, el, rng);
+  TrackIn in = LoadTrackIn(t, n, i);
+  const MscIn q = LoadMscIn(t, i);
+  KeepLoaded(in);
+  InitElectron(in, q, seed, el, rng);
   StepLoop<R> L;
   SlabPos p{s.x[i], g.plane[l], g.plane[l + 1], l == 0, l == g.nbins - 1, 0};
   const uint8_t f0 = s.lp.flags[i];
@@ -342,8 +379,10 @@ __device__ __forceinline__ void ElectronSubstep(const Stack& s, const Slabs& g, 
   const bool done = SlabSubstep(T, el, L, rng, p);
   const R rangeLeft = el.range;
   t.on_boundary[i] = p.side != 0 ? 1 : 0;
-  xend[i] = p.x;
-  side[i] = (int8_t)p.side;
+  mv.x = p.x;
+  mv.layer = l;
+  mv.side = p.side;
+  mv.ended = done;
   {
     const Msc<R>& m = el.msc;
     t.msc_init_range[i] = (double)m.initRange;
@@ -354,12 +393,12 @@ __device__ __forceinline__ void ElectronSubstep(const Stack& s, const Slabs& g, 
   SecList<R> sl;
   sl.ns = 0;
   double edep = 0.0;
+  uint8_t proc = kPNone;
   if (done) {
     L.preLEkin = L.preEkin > 0. ? vlog((R)L.preEkin) : (R)-30;
     s.lp.flags[i] = 0;
-    const int proc = LoopFinishSelect(T, el, L, sl, rng);
+    proc = ElectronProc(T, el.t, LoopFinishSelect(T, el, L, sl, rng));
     edep = el.t.edep;
-    ElectronFinalState(T, el.t, proc, sl, rng);
   } else {
     s.lp.range[i] = (double)rangeLeft;
     s.lp.stepLeft[i] = (double)L.stepLeft;
@@ -367,38 +406,38 @@ __device__ __forceinline__ void ElectronSubstep(const Stack& s, const Slabs& g, 
     s.lp.nsub[i] = L.nsub;
     s.lp.flags[i] = (uint8_t)(kInStep | kCont);
   }
-  res.edep[i] = edep;
 #pragma unroll
   for (int k = 0; k < 4; ++k) t.num_ia_left[k * n + i] = (double)el.t.nial[k];
-  t.ekin[i] = el.t.ekin;
-#pragma unroll
-  for (int c = 0; c < 3; ++c) t.dir[c * n + i] = (double)el.t.dir[c];
-  StoreRng(t, i, rng);
-  WriteSecondaries(res, n, i, sl);
+  if (proc != kPNone) {
+    const double d[3] = {(double)el.t.dir[0], (double)el.t.dir[1], (double)el.t.dir[2]};
+    return StageTrack(st, j, proc, el.t.isEl, el.t.imc, in.id, in.stream, el.t.ekin, d, rng, edep);
+  }
+  StoreFinal(t, res, n, i, el.t, rng, sl, edep, st[j]);
+  return kPNone;
 }
 
 // One step of gamma slot i, as G4HepEmTrackingManager::TrackGamma
 // takes it (G4HepEmTrackingManager.cc:893-1145): HowFar, the cut at the next
 // plane along x (or, with Woodcock tracking on and above its energy limit, a
 // Woodcock step through the stack), then the boundary update or
-// SelectInteraction + Perform. xend and side as ElectronSubstep; layer = the slab
-// the step's deposit is scored in (changed only by a Woodcock step).
+// SelectInteraction. The pending interaction as ElectronSubstep's (pe = the PE
+// cross section); the slab of the deposit is changed only by a Woodcock step.
 template <typename R, bool kWoodcock>
-__device__ __forceinline__ void GammaStep(const Stack& s, const Slabs& g, const hepem_step_out& res,
-                                          double* __restrict__ xend, int8_t* __restrict__ side,
-                                          const hepem::DevTables<R>& T, uint64_t seed, int i) {
+__device__ __forceinline__ uint8_t GammaStep(const Stack& s, const Slabs& g, const hepem_step_out& res,
+                                             const hepem::DevTables<R>& T, uint64_t seed, int i, Moved& mv, hepem::Staged* st,
+                                             int j) {
   using namespace hepem;
   const int n = s.t.n;
   hepem_tracks t = s.t;
   int l = s.layer[i];
   const double x = s.x[i];
-  SecList<R> sl;
-  sl.ns = 0;
   Trk<R> gt;
   gt.isEl = false;
-  LoadTrack(t, n, i, gt);
+  TrackIn in = LoadTrackIn(t, n, i);
+  KeepLoaded(in);
+  InitTrack(in, gt);
   Rng rng;
-  rng.init(seed, (uint32_t)t.id[i], StreamHi(t, i), t.rng_ctr[i], t.rng_has_gauss[i] != 0, t.rng_gauss[i]);
+  InitRng(in, seed, rng);
   R pe = GammaHowFar(T, gt, rng);
   const double ux = (double)gt.dir[0];
   double xe;
@@ -426,86 +465,131 @@ __device__ __forceinline__ void GammaStep(const Stack& s, const Slabs& g, const 
     s.layer[i] = l;
     t.imc[i] = gt.imc;
   }
-  GammaPerform(T, gt, pe, sl, rng);
-  t.ekin[i] = gt.ekin;
-#pragma unroll
-  for (int c = 0; c < 3; ++c) t.dir[c * n + i] = (double)gt.dir[c];
+  const uint8_t proc = GammaProc(T, gt, pe, rng);
   t.num_ia_left[i] = (double)gt.nial[0];
-  StoreRng(t, i, rng);
   t.on_boundary[i] = gt.onBoundary ? 1 : 0;
-  res.edep[i] = gt.edep;
-  WriteSecondaries(res, n, i, sl);
-  xend[i] = xe;
-  side[i] = (int8_t)sd;
-}
-
-// One sub-step of the e-/e+ slots [0, ne) in the first `ge` blocks and one step
-// of the gamma slots [ne, n) in the others. Bound by the latency of one wave's
-// chain as long as a round leaves most SIMDs with a wave or two of each kind:
-// in one launch the gamma waves run beside the e-/e+ waves instead of after
-// them, and an e-/e+ whose step ends goes on with its state in registers. Per
-// round of 1000 showers 73 us, against 38 for the sub-steps, 36 for the steps'
-// ends and 32 for the gammas in kernels of their own. Held to the waves per
-// SIMD that those kernels had (3 in FP64, 4 in the FP32-table form).
-template <typename R, bool kWoodcock>
-__global__ void __launch_bounds__(kB, sizeof(R) == sizeof(double) ? 3 : 4) k_sh_move(Stack s, Slabs g, hepem_step_out res, double* __restrict__ xend,
-                                                int8_t* __restrict__ side, hepem::DevTables<R> T, uint64_t seed, int ne,
-                                                int ge) {
-  if ((int)blockIdx.x < ge) {
-    const int i = (int)blockIdx.x * kB + (int)threadIdx.x;
-    if (i < ne) ElectronSubstep(s, g, res, xend, side, T, seed, i);
-  } else {
-    const int i = ne + ((int)blockIdx.x - ge) * kB + (int)threadIdx.x;
-    if (i < s.t.n) GammaStep<R, kWoodcock>(s, g, res, xend, side, T, seed, i);
+  mv.x = xe;
+  mv.layer = l;
+  mv.side = sd;
+  mv.ended = true;
+  if (proc != kPNone) {
+    const double d[3] = {(double)gt.dir[0], (double)gt.dir[1], (double)gt.dir[2]};
+    return StageTrack(st, j, proc, false, gt.imc, in.id, in.stream, gt.ekin, d, rng, (double)pe);
   }
+  SecList<R> sl;
+  sl.ns = 0;
+  StoreFinal(t, res, n, i, gt, rng, sl, 0.0, st[j]);
+  return kPNone;
 }
 
-// After Perform: position, slab crossing, scoring and next-round slot counts.
-// The next stack holds the e-/e+ first and the gammas after them (so the
-// library's particle-type queue covers runs of consecutive slots), each part
-// in slot order of the parents. keep[i] = 1 if the track itself goes on,
-// bit s of smask[i] = secondary slot s is stacked; offE/offG[i] = exclusive scans within the
-// block of the e-/e+ and gamma slots track i needs; bsumE/bsumG/bsec[block] =
-// the block's totals of those and of its secondaries. Deposits are summed per
-// block and (event, slab) before the global atomic; the fixed-point sum does
-// not depend on the grouping.
-__global__ void __launch_bounds__(kB) k_sh_post(Stack s, Slabs g, hepem_step_out res, const double* __restrict__ xend,
-                          const int8_t* __restrict__ side, unsigned long long* dep, unsigned long long* leak,
-                          uint8_t* keep, uint8_t* smask, uint32_t* offE, uint32_t* offG, uint32_t* bsumE, uint32_t* bsumG,
-                          uint32_t* bsec) {
-  const int i = blockIdx.x * kB + threadIdx.x;
+// Block -> slots of a round's stack: the e-/e+ slots [0, ne) in the first `ge`
+// blocks, the gammas after them in the others. i = the block's first slot; the
+// slots of its kind end before the returned one.
+__device__ __forceinline__ int BlockSlots(int n, int ne, int ge, int& i0) {
+  const bool isE = (int)blockIdx.x < ge;
+  i0 = isE ? (int)blockIdx.x * kB : ne + ((int)blockIdx.x - ge) * kB;
+  return isE ? ne : n;
+}
+
+// One sub-step of the e-/e+ slots and one step of the gammas (blocks as
+// BlockSlots), the final states of the interactions they end in, and the end of
+// the round for the block's slots.
+//
+// Bound by the latency of one wave's chain as long as a round leaves most SIMDs
+// with a wave or two, by VALU issue in the largest rounds. In one launch the
+// gamma waves run beside the e-/e+ waves instead of after them, and an e-/e+
+// whose step ends goes on with its state in registers. The final states are
+// sampled by process within the block: a wave with lanes in several processes
+// would run their samplers one after the other. The end of the round (a kernel
+// of its own read back ten arrays that this one had just written) takes the
+// position from registers and the rest from LDS. 1000 showers: 38.1 ms with the
+// sorted final states instead of 38.7, 35.1 instead of 36.5 without the kernel
+// that ended the round. Held to 3 waves per SIMD in FP64, 4 in the FP32-table
+// form.
+//
+// End of the round. The next stack holds the e-/e+ first and the gammas after
+// them, each part in slot order of the parents. next[i]: bit s = secondary slot
+// s is stacked, kSurvives = the track itself goes on; offE/offG[i] = exclusive
+// scans within the block of the e-/e+ and gamma slots track i needs;
+// bsumE/bsumG/bsec[block] = the block's totals of those and of its secondaries
+// (with the steps that ended in bits 16 and up). Deposits are summed per block
+// and (event, slab) before the global atomic; the fixed-point sum does not
+// depend on the grouping.
+constexpr uint8_t kSurvives = 4;
+constexpr int kHash = 2 * kB;
+template <typename R, bool kWoodcock>
+__global__ void __launch_bounds__(kB, sizeof(R) == sizeof(double) ? 3 : 4)
+    k_sh_move(Stack s, Slabs g, hepem_step_out res, hepem::DevTables<R> T, uint64_t seed, int ne, int ge, unsigned long long* dep,
+              unsigned long long* leak, uint8_t* __restrict__ next, uint32_t* __restrict__ offE, uint32_t* __restrict__ offG,
+              uint32_t* __restrict__ bsumE, uint32_t* __restrict__ bsumG, uint32_t* __restrict__ bsec) {
+  using namespace hepem;
+  __shared__ union {
+    BlockFinals<kB> fin;
+    struct {
+      unsigned long long key[kHash], val[kHash];
+    } hash;
+  } sh;
   const int n = s.t.n;
-  const bool valid = i < n;
-  const hepem_tracks& t = s.t;
-  // the steps that ended this round (an e-/e+ within its sub-steps has not),
-  // summed with the block's stacked secondaries in bsec (bits 16 and up)
-  const uint32_t ended = (valid && (t.ptype[i] == 2 || !(s.lp.flags[i] & kInStep))) ? 1u : 0u;
+  hepem_tracks t = s.t;
+  int i0;
+  const int last = BlockSlots(n, ne, ge, i0), i = i0 + (int)threadIdx.x;
+  const bool valid = i < last, isE = (int)blockIdx.x < ge;
+  uint8_t code = kPNone;
+  Moved mv;
+  if (isE) {
+    if (valid) code = ElectronSubstep(s, g, res, T, seed, i, mv, sh.fin.st, (int)threadIdx.x);
+    SampleBlock<kB, kPIoniEl, kPAnnih>(sh.fin, code, [&](int j, Staged& r, uint8_t c, int proc) {
+      Trk<R> k;
+      Rng rng;
+      SecList<R> sl;
+      sl.ns = 0;
+      const double edep = r.pe;
+      Unstage(r, c, seed, k, rng);
+      ElectronFinal(T, k, proc, sl, rng);
+      StoreFinal(t, res, n, i0 + j, k, rng, sl, edep, r);
+    });
+  } else {
+    if (valid) code = GammaStep<R, kWoodcock>(s, g, res, T, seed, i, mv, sh.fin.st, (int)threadIdx.x);
+    SampleBlock<kB, kPConv, kPPE>(sh.fin, code, [&](int j, Staged& r, uint8_t c, int proc) {
+      Trk<R> k;
+      Rng rng;
+      SecList<R> sl;
+      sl.ns = 0;
+      const R pe = (R)r.pe;
+      Unstage(r, c, seed, k, rng);
+      GammaFinal(T, k, proc, pe, sl, rng);
+      StoreFinal(t, res, n, i0 + j, k, rng, sl, k.edep, r);
+    });
+  }
+  __syncthreads();
+  const Staged r = sh.fin.st[threadIdx.x];
+  __syncthreads();  // the hash table takes the records' place
+  const uint32_t ended = valid && mv.ended ? 1u : 0u;
   constexpr unsigned long long kNone = ~0ull;
   unsigned long long key = kNone, val = 0ull;
   uint32_t cE = 0u, cG = 0u, ns = 0u;
   if (valid) {
     const int ev = s.event[i];
-    const int l0 = s.layer[i];  // the pre-step slab: scoring and the couple's cuts
+    const int l0 = mv.layer;  // the pre-step slab: scoring and the couple's cuts
     int l = l0;
-    double edep = res.edep[i];
-    const double x = xend[i];
-    const int sd = side[i];
-    const bool isE = t.ptype[i] != 2;
-    const double ekin = t.ekin[i];
+    const double ekin = r.ekin;
+    double edep = r.dir[0];
+    const int sd = mv.side;
     bool alive = ekin > 0.0;
-    int nsec = res.nsec[i];
+    int nsec = r.imc;
     if (sd != 0 && (l + sd < 0 || l + sd >= g.nbins)) {
       // leaves the stack: its kinetic energy, the annihilation energy of an e+
       // in flight and anything its last step created are lost
       double e = ekin + (t.ptype[i] == 1 && ekin > 0.0 ? 2.0 * kElectronMass : 0.0);
-      for (int sl = 0; sl < nsec; ++sl) e += res.sec_ekin[sl * n + i];
+      if (nsec > 0) e += r.dir[1];
+      if (nsec > 1) e += r.dir[2];
       atomicAdd(&leak[ev], (unsigned long long)llrint(e * kFix));
       alive = false;
       nsec = 0;
     } else if (alive && sd != 0) {
       l += sd;
     }
-    s.x[i] = x;
+    s.x[i] = mv.x;
     s.layer[i] = l;
     // StackSecondaries (G4HepEmTrackingManager.cc:1274-1313): where the
     // couple's region applies cuts, a secondary below its production
@@ -513,9 +597,11 @@ __global__ void __launch_bounds__(kB) k_sh_post(Stack s, Slabs g, hepem_step_out
     // annihilation energy, when the gamma threshold exceeds the electron mass)
     const int a = l0 % g.nabs;
     uint32_t mask = 0u;
-    for (int sl = 0; sl < nsec; ++sl) {
-      const int8_t pt = res.sec_ptype[sl * n + i];
-      const double se = res.sec_ekin[sl * n + i];
+#pragma unroll
+    for (int sl = 0; sl < 2; ++sl) {
+      if (sl >= nsec) continue;
+      const int pt = sl ? (int)r.stream : r.id;
+      const double se = sl ? r.dir[2] : r.dir[1];
       bool cut = false;
       if (g.applyCuts[a]) {
         if (pt == 0) cut = se < g.cutE[a];
@@ -531,8 +617,7 @@ __global__ void __launch_bounds__(kB) k_sh_post(Stack s, Slabs g, hepem_step_out
         else ++cE;
       }
     }
-    keep[i] = alive ? 1 : 0;
-    smask[i] = (uint8_t)mask;
+    next[i] = (uint8_t)(mask | (alive ? kSurvives : 0));
     if (alive) {
       if (isE) ++cE;
       else ++cG;
@@ -545,19 +630,17 @@ __global__ void __launch_bounds__(kB) k_sh_post(Stack s, Slabs g, hepem_step_out
   // per-block aggregation of the deposits in an LDS hash table (open
   // addressing, at most kB keys in 2 kB entries, so every probe sequence ends):
   // one global atomic per distinct (event, slab) of the block
-  constexpr int kHash = 2 * kB;
-  __shared__ unsigned long long hkey[kHash], hval[kHash];
   for (int e = threadIdx.x; e < kHash; e += kB) {
-    hkey[e] = kNone;
-    hval[e] = 0ull;
+    sh.hash.key[e] = kNone;
+    sh.hash.val[e] = 0ull;
   }
   __syncthreads();
   if (key != kNone) {
     uint32_t h = (uint32_t)((key * 0x9E3779B97F4A7C15ull) >> 55) & (kHash - 1);
     while (true) {
-      const unsigned long long prev = atomicCAS(&hkey[h], kNone, key);
+      const unsigned long long prev = atomicCAS(&sh.hash.key[h], kNone, key);
       if (prev == kNone || prev == key) {
-        atomicAdd(&hval[h], val);
+        atomicAdd(&sh.hash.val[h], val);
         break;
       }
       h = (h + 1) & (kHash - 1);
@@ -565,8 +648,8 @@ __global__ void __launch_bounds__(kB) k_sh_post(Stack s, Slabs g, hepem_step_out
   }
   __syncthreads();
   for (int e = threadIdx.x; e < kHash; e += kB) {
-    const unsigned long long k = hkey[e];
-    if (k != kNone) atomicAdd(&dep[k], hval[e]);
+    const unsigned long long k = sh.hash.key[e];
+    if (k != kNone) atomicAdd(&dep[k], sh.hash.val[e]);
   }
   uint32_t xE, xG, tE, tG, tns;
   hepem::BlockScan2<kB>(cE, cG, ns | (ended << 16), xE, xG, tE, tG, tns);
@@ -646,13 +729,14 @@ __global__ void __launch_bounds__(kScanB) k_scan_sums(uint32_t* bsumE, uint32_t*
 // bsumG[block] + offG[i], in the order survivor, secondary 0, secondary 1;
 // each starts with the isotropic safety of its position. Writes nothing beyond
 // `cap` (the host then reports the overflow).
-__global__ void __launch_bounds__(kB) k_sh_scatter(Stack a, Stack b, Slabs g, hepem_step_out res, const uint8_t* __restrict__ keep,
-                             const uint8_t* __restrict__ smask, const uint32_t* __restrict__ offE,
+__global__ void __launch_bounds__(kB) k_sh_scatter(Stack a, Stack b, Slabs g, hepem_step_out res, int ne, int ge,
+                             const uint8_t* __restrict__ next, const uint32_t* __restrict__ offE,
                              const uint32_t* __restrict__ offG, const uint32_t* __restrict__ bsumE,
                              const uint32_t* __restrict__ bsumG, const uint32_t* __restrict__ total, int cap) {
-  const int i = blockIdx.x * kB + threadIdx.x;
   const int n = a.t.n;
-  if (i >= n) return;
+  int i0;
+  const int last = BlockSlots(n, ne, ge, i0), i = i0 + (int)threadIdx.x;
+  if (i >= last) return;
   const int m = (int)total[0];
   if (m > cap) return;
   const hepem_tracks& s = a.t;
@@ -668,7 +752,8 @@ __global__ void __launch_bounds__(kB) k_sh_scatter(Stack a, Stack b, Slabs g, he
   // neither the safety nor the MSC state: those fields of a gamma slot are not
   // carried (the e-/e+ and gamma parts of the stack keep whole waves on one
   // side of these branches).
-  if (keep[i]) {
+  const uint32_t mask = next[i];
+  if (mask & kSurvives) {
     const int8_t pt = s.ptype[i];
     const bool isE = pt != 2;
     const int j = isE ? jE++ : jG++;
@@ -712,7 +797,6 @@ __global__ void __launch_bounds__(kB) k_sh_scatter(Stack a, Stack b, Slabs g, he
     b.event[j] = a.event[i];
     b.nstep[j] = inStep ? a.nstep[i] : ns1;  // a step counts once it ends
   }
-  const uint32_t mask = smask[i];
   for (int sl = 0; sl < 2; ++sl) {
     if (!((mask >> sl) & 1u)) continue;
     const uint64_t cid = ChildStream(sid, ns1, sl);
@@ -893,30 +977,26 @@ extern "C" int hepem_slab_run(const hepem_ctx* ctx, const hepem_slab_setup* su, 
 
   Arena A;
   Stack s[2];
-  hepem_step_out res;  // the fields the stepping kernel writes and the post kernel reads
+  hepem_step_out res;  // the secondaries, from the stepping kernel to the scatter
   res.true_step = nullptr;
   res.geom_step = nullptr;
   res.winner = nullptr;
   res.displacement = nullptr;
   res.stopped = nullptr;
-  double *dPlanes, *xend;
-  int8_t* side;
-  uint8_t *keep, *smask;
+  res.edep = nullptr;
+  res.nsec = nullptr;
+  double* dPlanes;
+  uint8_t* goesOn;
   uint32_t *offs, *bsum, *bsec, *total;  // offs: e-/e+ then gamma block offsets (2 x cap); bsum: 2 x nblk
   unsigned long long *dep, *leak, *nsec;
-  const int nblk = (cap + kB - 1) / kB;
+  const int nblk = (cap + kB - 1) / kB + 1;  // the e-/e+ and the gamma part of a round each end with a block
   AskStack(A, s[0], (size_t)cap);
   AskStack(A, s[1], (size_t)cap);
-  A.get(res.edep, (size_t)cap);
-  A.get(res.nsec, (size_t)cap);
   A.get(res.sec_ptype, 2 * (size_t)cap);
   A.get(res.sec_ekin, 2 * (size_t)cap);
   A.get(res.sec_dir, 6 * (size_t)cap);
   A.get(dPlanes, planes.size());
-  A.get(xend, (size_t)cap);
-  A.get(side, (size_t)cap);
-  A.get(keep, (size_t)cap);
-  A.get(smask, (size_t)cap);
+  A.get(goesOn, (size_t)cap);
   A.get(offs, 2 * (size_t)cap);
   A.get(bsum, 2 * (size_t)nblk);
   A.get(bsec, (size_t)nblk);
@@ -1019,20 +1099,21 @@ extern "C" int hepem_slab_run(const hepem_ctx* ctx, const hepem_slab_setup* su, 
       Stack& a = s[cur];
       Stack& b = s[cur ^ 1];
       a.t.n = n;
-      const int grid = (n + kB - 1) / kB;
       // the e-/e+ part of the stack comes first
       const int ge = (ne + kB - 1) / kB, gg = (n - ne + kB - 1) / kB;
       if (fp64 && woodcock)
-        hipLaunchKernelGGL((k_sh_move<double, true>), dim3(ge + gg), dim3(kB), 0, st, a, g, res, xend, side, HepemTables64(ctx), seed, ne, ge);
+        hipLaunchKernelGGL((k_sh_move<double, true>), dim3(ge + gg), dim3(kB), 0, st, a, g, res, HepemTables64(ctx), seed, ne, ge, dep,
+                           leak, goesOn, offs, offs + cap, bsum, bsum + nblk, bsec);
       else if (fp64)
-        hipLaunchKernelGGL((k_sh_move<double, false>), dim3(ge + gg), dim3(kB), 0, st, a, g, res, xend, side, HepemTables64(ctx), seed, ne, ge);
+        hipLaunchKernelGGL((k_sh_move<double, false>), dim3(ge + gg), dim3(kB), 0, st, a, g, res, HepemTables64(ctx), seed, ne, ge, dep,
+                           leak, goesOn, offs, offs + cap, bsum, bsum + nblk, bsec);
       else if (woodcock)
-        hipLaunchKernelGGL((k_sh_move<float, true>), dim3(ge + gg), dim3(kB), 0, st, a, g, res, xend, side, HepemTables32(ctx), seed, ne, ge);
+        hipLaunchKernelGGL((k_sh_move<float, true>), dim3(ge + gg), dim3(kB), 0, st, a, g, res, HepemTables32(ctx), seed, ne, ge, dep,
+                           leak, goesOn, offs, offs + cap, bsum, bsum + nblk, bsec);
       else
-        hipLaunchKernelGGL((k_sh_move<float, false>), dim3(ge + gg), dim3(kB), 0, st, a, g, res, xend, side, HepemTables32(ctx), seed, ne, ge);
+        hipLaunchKernelGGL((k_sh_move<float, false>), dim3(ge + gg), dim3(kB), 0, st, a, g, res, HepemTables32(ctx), seed, ne, ge, dep,
+                           leak, goesOn, offs, offs + cap, bsum, bsum + nblk, bsec);
       r->substeps += ne;
-      hipLaunchKernelGGL(k_sh_post, dim3(grid), dim3(kB), 0, st, a, g, res, xend, side, dep, leak, keep, smask, offs, offs + cap,
-                         bsum, bsum + nblk, bsec);
       // primaries of the next events join once the stack runs low, and no
       // sooner after the last ones than the first events took to reach their
       // largest stack: the stack then stays below about refill plus one chunk's
@@ -1040,10 +1121,10 @@ extern "C" int hepem_slab_run(const hepem_ctx* ctx, const hepem_slab_setup* su, 
       const bool refillNow = refill > 0 && n < refill && next < ns && growRounds >= 0 && sinceInject >= growRounds;
       const int k = refillNow ? ((ns - next) < chunk ? (ns - next) : chunk) : 0;
       ++tag;
-      hipLaunchKernelGGL(k_scan_sums, dim3(1), dim3(kScanB), 0, st, bsum, bsum + nblk, bsec, grid, k, su->primary != 2 ? 1 : 0,
+      hipLaunchKernelGGL(k_scan_sums, dim3(1), dim3(kScanB), 0, st, bsum, bsum + nblk, bsec, ge + gg, k, su->primary != 2 ? 1 : 0,
                          total, nsec, nsec + 1, hc.d, tag);
-      hipLaunchKernelGGL(k_sh_scatter, dim3(grid), dim3(kB), 0, st, a, b, g, res, keep, smask, offs, offs + cap, bsum, bsum + nblk,
-                         total, cap);
+      hipLaunchKernelGGL(k_sh_scatter, dim3(ge + gg), dim3(kB), 0, st, a, b, g, res, ne, ge, goesOn, offs, offs + cap, bsum,
+                         bsum + nblk, total, cap);
       if (k > 0) {
         hipLaunchKernelGGL(k_sh_inject, dim3((k + kB - 1) / kB), dim3(kB), 0, st, b, g, su->primary, su->ekin0,
                            (int)(s0 + next), next, k, total + 1, total, cap);
