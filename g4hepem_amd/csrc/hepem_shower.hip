@@ -729,6 +729,17 @@ __global__ void __launch_bounds__(kScanB) k_scan_sums(uint32_t* bsumE, uint32_t*
 // bsumG[block] + offG[i], in the order survivor, secondary 0, secondary 1;
 // each starts with the isotropic safety of its position. Writes nothing beyond
 // `cap` (the host then reports the overflow).
+//
+// Bound by latency in small rounds, by its bytes in large ones. Everything is
+// loaded before the first store: the arrays may overlap as far as the compiler
+// knows, so copied field by field each load waited for the one before it to be
+// stored (1000 showers 35.1 ms, now 33.3).
+struct ElSlot {  // what an e-/e+ slot carries beyond a gamma's
+  double nial[3], initRange, dynRangeFactor, tlimitMin, safety, range, stepLeft, mfp[4], preEkin, meanLoss;
+  int32_t nsub;
+  int8_t iDProc;
+  uint8_t firstStep, flags;
+};
 __global__ void __launch_bounds__(kB) k_sh_scatter(Stack a, Stack b, Slabs g, hepem_step_out res, int ne, int ge,
                              const uint8_t* __restrict__ next, const uint32_t* __restrict__ offE,
                              const uint32_t* __restrict__ offG, const uint32_t* __restrict__ bsumE,
@@ -737,81 +748,114 @@ __global__ void __launch_bounds__(kB) k_sh_scatter(Stack a, Stack b, Slabs g, he
   int i0;
   const int last = BlockSlots(n, ne, ge, i0), i = i0 + (int)threadIdx.x;
   if (i >= last) return;
-  const int m = (int)total[0];
-  if (m > cap) return;
   const hepem_tracks& s = a.t;
   const hepem_tracks& d = b.t;
-  int jE = (int)(bsumE[blockIdx.x] + offE[i]);
-  int jG = (int)(total[2] + bsumG[blockIdx.x] + offG[i]);
-  const double x = a.x[i];
-  const int l = a.layer[i];
-  const double safety = Safety(g, l, x);
-  const uint64_t sid = ((uint64_t)s.rng_stream[i] << 32) | (uint32_t)s.id[i];
-  const int ns1 = a.nstep[i] + 1;
+  const bool isE = (int)blockIdx.x < ge;
   // A gamma reads only the first interaction-length slot (its total) and
   // neither the safety nor the MSC state: those fields of a gamma slot are not
-  // carried (the e-/e+ and gamma parts of the stack keep whole waves on one
-  // side of these branches).
+  // carried.
   const uint32_t mask = next[i];
+  const int m = (int)total[0];
+  int jE = (int)(bsumE[blockIdx.x] + offE[i]);
+  int jG = (int)(total[2] + bsumG[blockIdx.x] + offG[i]);
+  const double x = a.x[i], ekin = s.ekin[i], gauss = s.rng_gauss[i], nial0 = s.num_ia_left[i];
+  const double dir0 = s.dir[i], dir1 = s.dir[n + i], dir2 = s.dir[2 * n + i];
+  const int l = a.layer[i], ev = a.event[i], nstep = a.nstep[i];
+  const int32_t id = s.id[i];
+  const uint32_t stream = s.rng_stream[i], ctr = s.rng_ctr[i];
+  const int8_t pt = s.ptype[i];
+  const uint8_t onb = s.on_boundary[i], hasGauss = s.rng_has_gauss[i];
+  ElSlot e;
+  if (isE) {
+    for (int k = 0; k < 3; ++k) e.nial[k] = s.num_ia_left[(k + 1) * n + i];
+    e.initRange = s.msc_init_range[i];
+    e.dynRangeFactor = s.msc_dyn_range_factor[i];
+    e.tlimitMin = s.msc_tlimit_min[i];
+    e.firstStep = s.msc_first_step[i];
+    e.flags = a.lp.flags[i];
+    // within a step: its pre-step safety and the loop state go along
+    if ((mask & kSurvives) && (e.flags & kInStep)) {
+      e.safety = s.safety[i];
+      e.range = a.lp.range[i];
+      e.stepLeft = a.lp.stepLeft[i];
+      for (int k = 0; k < 4; ++k) e.mfp[k] = a.lp.mfp[k * n + i];
+      e.preEkin = a.lp.preEkin[i];
+      e.meanLoss = a.lp.meanLoss[i];
+      e.nsub = a.lp.nsub[i];
+      e.iDProc = a.lp.iDProc[i];
+    }
+  }
+  int8_t secType[2];
+  double secE[2], secDir[2][3];
+#pragma unroll
+  for (int sl = 0; sl < 2; ++sl) {
+    if (!((mask >> sl) & 1u)) continue;
+    secType[sl] = res.sec_ptype[sl * n + i];
+    secE[sl] = res.sec_ekin[sl * n + i];
+    for (int c = 0; c < 3; ++c) secDir[sl][c] = res.sec_dir[(c * 2 + sl) * n + i];
+  }
+  if (m > cap) return;
+  const double safety = Safety(g, l, x);
+  const int imc = AbsorberCouple(g, l % g.nabs);
+  const uint64_t sid = ((uint64_t)stream << 32) | (uint32_t)id;
+  const int ns1 = nstep + 1;
   if (mask & kSurvives) {
-    const int8_t pt = s.ptype[i];
-    const bool isE = pt != 2;
     const int j = isE ? jE++ : jG++;
     d.ptype[j] = pt;
-    d.id[j] = s.id[i];
-    d.rng_stream[j] = s.rng_stream[i];
-    d.imc[j] = g.imc[l % g.nabs];
-    d.ekin[j] = s.ekin[i];
-    for (int c = 0; c < 3; ++c) d.dir[c * m + j] = s.dir[c * n + i];
-    d.on_boundary[j] = s.on_boundary[i];
-    d.num_ia_left[j] = s.num_ia_left[i];
+    d.id[j] = id;
+    d.rng_stream[j] = stream;
+    d.imc[j] = imc;
+    d.ekin[j] = ekin;
+    d.dir[j] = dir0;
+    d.dir[m + j] = dir1;
+    d.dir[2 * m + j] = dir2;
+    d.on_boundary[j] = onb;
+    d.num_ia_left[j] = nial0;
     bool inStep = false;
     if (isE) {
-      for (int k = 1; k < 4; ++k) d.num_ia_left[k * m + j] = s.num_ia_left[k * n + i];
-      d.msc_init_range[j] = s.msc_init_range[i];
-      d.msc_dyn_range_factor[j] = s.msc_dyn_range_factor[i];
-      d.msc_tlimit_min[j] = s.msc_tlimit_min[i];
-      d.msc_first_step[j] = s.msc_first_step[i];
-      const uint8_t f = a.lp.flags[i];
-      inStep = (f & kInStep) != 0;
-      b.lp.flags[j] = inStep ? f : (uint8_t)0;
+      for (int k = 0; k < 3; ++k) d.num_ia_left[(k + 1) * m + j] = e.nial[k];
+      d.msc_init_range[j] = e.initRange;
+      d.msc_dyn_range_factor[j] = e.dynRangeFactor;
+      d.msc_tlimit_min[j] = e.tlimitMin;
+      d.msc_first_step[j] = e.firstStep;
+      inStep = (e.flags & kInStep) != 0;
+      b.lp.flags[j] = inStep ? e.flags : (uint8_t)0;
       if (inStep) {
-        // within a step: its pre-step safety and the loop state go along
-        d.safety[j] = s.safety[i];
-        b.lp.range[j] = a.lp.range[i];
-        b.lp.stepLeft[j] = a.lp.stepLeft[i];
-        for (int k = 0; k < 4; ++k) b.lp.mfp[k * m + j] = a.lp.mfp[k * n + i];
-        b.lp.preEkin[j] = a.lp.preEkin[i];
-        b.lp.meanLoss[j] = a.lp.meanLoss[i];
-        b.lp.nsub[j] = a.lp.nsub[i];
-        b.lp.iDProc[j] = a.lp.iDProc[i];
+        d.safety[j] = e.safety;
+        b.lp.range[j] = e.range;
+        b.lp.stepLeft[j] = e.stepLeft;
+        for (int k = 0; k < 4; ++k) b.lp.mfp[k * m + j] = e.mfp[k];
+        b.lp.preEkin[j] = e.preEkin;
+        b.lp.meanLoss[j] = e.meanLoss;
+        b.lp.nsub[j] = e.nsub;
+        b.lp.iDProc[j] = e.iDProc;
       } else {
         d.safety[j] = safety;
       }
     }
-    d.rng_ctr[j] = s.rng_ctr[i];
-    d.rng_gauss[j] = s.rng_gauss[i];
-    d.rng_has_gauss[j] = s.rng_has_gauss[i];
+    d.rng_ctr[j] = ctr;
+    d.rng_gauss[j] = gauss;
+    d.rng_has_gauss[j] = hasGauss;
     b.x[j] = x;
     b.layer[j] = l;
-    b.event[j] = a.event[i];
-    b.nstep[j] = inStep ? a.nstep[i] : ns1;  // a step counts once it ends
+    b.event[j] = ev;
+    b.nstep[j] = inStep ? nstep : ns1;  // a step counts once it ends
   }
+#pragma unroll
   for (int sl = 0; sl < 2; ++sl) {
     if (!((mask >> sl) & 1u)) continue;
     const uint64_t cid = ChildStream(sid, ns1, sl);
-    const int8_t pt = res.sec_ptype[sl * n + i];
-    const bool isE = pt != 2;
-    const int j = isE ? jE++ : jG++;
-    d.ptype[j] = pt;
+    const bool secIsE = secType[sl] != 2;
+    const int j = secIsE ? jE++ : jG++;
+    d.ptype[j] = secType[sl];
     d.id[j] = (int32_t)(uint32_t)cid;
     d.rng_stream[j] = (uint32_t)(cid >> 32);
-    d.imc[j] = g.imc[l % g.nabs];
-    d.ekin[j] = res.sec_ekin[sl * n + i];
-    for (int c = 0; c < 3; ++c) d.dir[c * m + j] = res.sec_dir[(c * 2 + sl) * n + i];
+    d.imc[j] = imc;
+    d.ekin[j] = secE[sl];
+    for (int c = 0; c < 3; ++c) d.dir[c * m + j] = secDir[sl][c];
     d.on_boundary[j] = 0;
     d.num_ia_left[j] = -1.0;
-    if (isE) {
+    if (secIsE) {
       d.safety[j] = safety;
       b.lp.flags[j] = 0;
       for (int k = 1; k < 4; ++k) d.num_ia_left[k * m + j] = -1.0;
@@ -825,7 +869,7 @@ __global__ void __launch_bounds__(kB) k_sh_scatter(Stack a, Stack b, Slabs g, he
     d.rng_has_gauss[j] = 0;
     b.x[j] = x;
     b.layer[j] = l;
-    b.event[j] = a.event[i];
+    b.event[j] = ev;
     b.nstep[j] = 0;
   }
 }
