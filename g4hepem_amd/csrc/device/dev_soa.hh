@@ -284,22 +284,54 @@ template <typename R> HD void StoreElectronHowFar(const hepem_howfar_state& hs, 
   hs.msc_active[i] = m.active ? 1 : 0;
   hs.msc_displace[i] = m.isDisplace ? 1 : 0;
 }
-template <typename R> HD void LoadElectronHowFar(const hepem_howfar_state& hs, int n, int i, ElState<R>& el) {
+// The hand-over as loaded.
+struct HowFarIn {
+  double gstep, range, mfp[4], lambtr1, trueStep, zpath, par1, par2, par3;
+  int winner;
+  uint8_t active, displace;
+};
+HD HowFarIn LoadHowFarIn(const hepem_howfar_state& hs, int n, int i) {
+  HowFarIn h;
+  h.gstep = hs.geom_step[i];
+  h.range = hs.range[i];
+#pragma unroll
+  for (int k = 0; k < 4; ++k) h.mfp[k] = hs.mfp[k * n + i];
+  h.winner = hs.winner[i];
+  h.lambtr1 = hs.msc_lambtr1[i];
+  h.trueStep = hs.msc_true_step[i];
+  h.zpath = hs.msc_zpath[i];
+  h.par1 = hs.msc_par1[i];
+  h.par2 = hs.msc_par2[i];
+  h.par3 = hs.msc_par3[i];
+  h.active = hs.msc_active[i];
+  h.displace = hs.msc_displace[i];
+  return h;
+}
+HD void KeepLoaded(HowFarIn& h) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  asm volatile("" : "+v"(h.gstep), "+v"(h.range), "+v"(h.mfp[0]), "+v"(h.mfp[1]), "+v"(h.mfp[2]), "+v"(h.mfp[3]), "+v"(h.lambtr1),
+               "+v"(h.trueStep), "+v"(h.zpath), "+v"(h.par1), "+v"(h.par2), "+v"(h.par3), "+v"(h.winner));
+#endif
+}
+template <typename R> HD void SetHowFar(const HowFarIn& h, ElState<R>& el) {
   Trk<R>& t = el.t;
   Msc<R>& m = el.msc;
-  t.gstep = (R)hs.geom_step[i];
-  el.range = (R)hs.range[i];
+  t.gstep = (R)h.gstep;
+  el.range = (R)h.range;
 #pragma unroll
-  for (int k = 0; k < 4; ++k) t.mfp[k] = (R)hs.mfp[k * n + i];
-  t.winner = hs.winner[i];
-  m.lambtr1 = (R)hs.msc_lambtr1[i];
-  m.trueStep = (R)hs.msc_true_step[i];
-  m.zpath = (R)hs.msc_zpath[i];
-  m.par1 = (R)hs.msc_par1[i];
-  m.par2 = (R)hs.msc_par2[i];
-  m.par3 = (R)hs.msc_par3[i];
-  m.active = hs.msc_active[i] != 0;
-  m.isDisplace = hs.msc_displace[i] != 0;
+  for (int k = 0; k < 4; ++k) t.mfp[k] = (R)h.mfp[k];
+  t.winner = h.winner;
+  m.lambtr1 = (R)h.lambtr1;
+  m.trueStep = (R)h.trueStep;
+  m.zpath = (R)h.zpath;
+  m.par1 = (R)h.par1;
+  m.par2 = (R)h.par2;
+  m.par3 = (R)h.par3;
+  m.active = h.active != 0;
+  m.isDisplace = h.displace != 0;
+}
+template <typename R> HD void LoadElectronHowFar(const hepem_howfar_state& hs, int n, int i, ElState<R>& el) {
+  SetHowFar(LoadHowFarIn(hs, n, i), el);
 }
 
 // G4HepEmElectronManager::HowFar + Perform (G4HepEmElectronManager.icc:35-45,

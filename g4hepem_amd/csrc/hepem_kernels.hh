@@ -129,17 +129,86 @@ __device__ inline void CountWave(uint32_t* c, bool pred) {
   if (m && __lane_id() == __ffsll((unsigned long long)m) - 1) atomicAdd(c, (uint32_t)__popcll(m));
 }
 
-template <typename R> HD void LoadLoop(const hepem_substep_state& ss, int i, StepLoop<R>& L) {
-  L.iDProc = ss.discrete_winner[i];
-  L.stepLeft = (R)ss.step_left[i];
-  L.truePath = (R)ss.true_path[i];
-  L.meanLoss = ss.mean_eloss[i];
-  L.preEkin = ss.pre_ekin[i];
+struct LoopIn {
+  double stepLeft, truePath, meanLoss, preEkin;
+  int iDProc, nsub;
+  uint8_t more, stopped, left;
+};
+HD LoopIn LoadLoopIn(const hepem_substep_state& ss, int i) {
+  LoopIn r;
+  r.iDProc = ss.discrete_winner[i];
+  r.stepLeft = ss.step_left[i];
+  r.truePath = ss.true_path[i];
+  r.meanLoss = ss.mean_eloss[i];
+  r.preEkin = ss.pre_ekin[i];
+  r.more = ss.more[i];
+  r.stopped = ss.stopped[i];
+  r.left = ss.left_world[i];
+  r.nsub = ss.nsub[i];
+  return r;
+}
+HD void KeepLoaded(LoopIn& r) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  asm volatile("" : "+v"(r.stepLeft), "+v"(r.truePath), "+v"(r.meanLoss), "+v"(r.preEkin), "+v"(r.iDProc), "+v"(r.nsub));
+#endif
+}
+template <typename R> HD void SetLoop(const LoopIn& r, StepLoop<R>& L) {
+  L.iDProc = r.iDProc;
+  L.stepLeft = (R)r.stepLeft;
+  L.truePath = (R)r.truePath;
+  L.meanLoss = r.meanLoss;
+  L.preEkin = r.preEkin;
   L.preLEkin = L.preEkin > 0. ? vlog((R)L.preEkin) : (R)-30;
-  L.cont = ss.more[i] != 0;
-  L.stopped = ss.stopped[i] != 0;
-  L.left = ss.left_world[i] != 0;
-  L.nsub = ss.nsub[i];
+  L.cont = r.more != 0;
+  L.stopped = r.stopped != 0;
+  L.left = r.left != 0;
+  L.nsub = r.nsub;
+}
+// The whole state of an e-/e+ slot between the calls, loaded at once (left to
+// itself the compiler moves loads down to the branches that use them, and the
+// wave waits for memory at each). With the active slots closed up (ActiveSlot)
+// and the end's final states sorted by process, 100k e-/e+ through 27 sub-steps
+// take 1.88 ms instead of 2.15: the along-step kernel 20 us instead of 32 (the
+// median of its sub-steps), the MSC HowFar 10 instead of 13, the end 41 instead
+// of 52.
+template <typename R>
+HD void LoadSubstep(const hepem_tracks& t, const hepem_howfar_state& hs, const hepem_substep_state& ss, int n, int i, uint64_t seed,
+                    ElState<R>& el, StepLoop<R>& L, Rng& rng) {
+  TrackIn r = LoadTrackIn(t, n, i);
+  const MscIn q = LoadMscIn(t, i);
+  HowFarIn h = LoadHowFarIn(hs, n, i);
+  LoopIn l = LoadLoopIn(ss, i);
+  KeepLoaded(r);
+  KeepLoaded(h);
+  KeepLoaded(l);
+  InitElectron(r, q, seed, el, rng);
+  SetHowFar(h, el);
+  SetLoop(l, L);
+}
+// The block's active slots, closed up: returns the slot of this thread (of the
+// block's active ones in slot order), or -1 past their number. After the first
+// sub-steps few slots of a wave still are within their step, and each wave with
+// one left runs its whole chain; closed up, a block's fit fewer waves.
+__device__ __forceinline__ int ActiveSlot(const uint8_t* __restrict__ active, int n) {
+  __shared__ uint32_t sCount[kWaves];
+  __shared__ uint8_t sSlot[kBlock];
+  static_assert(kBlock <= 256, "slots of a block are 8 bits");
+  const int lane = __lane_id(), wave = threadIdx.x >> 6;
+  const int i0 = blockIdx.x * kBlock, i = i0 + (int)threadIdx.x;
+  const bool act = i < n && active[i] != 0;
+  const uint64_t m = __ballot(act);
+  if (lane == 0) sCount[wave] = (uint32_t)__popcll(m);
+  __syncthreads();
+  uint32_t before = 0u, total = 0u;
+#pragma unroll
+  for (int w = 0; w < kWaves; ++w) {
+    const uint32_t c = sCount[w];
+    before += w < wave ? c : 0u;
+    total += c;
+  }
+  if (act) sSlot[before + (uint32_t)__popcll(m & ((1ull << lane) - 1ull))] = (uint8_t)threadIdx.x;
+  __syncthreads();
+  return threadIdx.x < total ? i0 + (int)sSlot[threadIdx.x] : -1;
 }
 template <typename R> HD void StoreLoop(const hepem_substep_state& ss, int i, const StepLoop<R>& L) {
   ss.discrete_winner[i] = L.iDProc;
@@ -189,16 +258,14 @@ __global__ void __launch_bounds__(kBlock) k_el_begin(DevTables<R> T, uint64_t se
 template <typename R>
 __global__ void __launch_bounds__(kBlock) k_el_substep_howfar(DevTables<R> T, uint64_t seed, hepem_tracks t,
                                                               hepem_howfar_state hs, hepem_substep_state ss) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
   const int n = t.n;
-  if (i >= n || !ss.active[i]) return;
+  const int i = ActiveSlot(ss.active, n);
+  if (i < 0) return;
   ElState<R> el;
   Rng rng;
-  InitElectron(t, n, i, seed, el, rng);
-  LoadElectronHowFar(hs, n, i, el);
-  el.pstep = (R)ss.step_left[i];
   StepLoop<R> L;
-  LoadLoop(ss, i, L);
+  LoadSubstep(t, hs, ss, n, i, seed, el, L, rng);
+  el.pstep = L.stepLeft;
   LoopMsc(T, el, L, rng);
   StoreElectronState(t, n, i, el, rng);
   StoreElectronHowFar(hs, n, i, el);
@@ -210,23 +277,22 @@ template <typename R>
 __global__ void __launch_bounds__(kBlock) k_el_substep_along(DevTables<R> T, uint64_t seed, hepem_tracks t,
                                                              hepem_howfar_state hs, hepem_substep_state ss,
                                                              uint32_t* __restrict__ counters) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
   const int n = t.n;
+  const int i = ActiveSlot(ss.active, n);
   bool again = false;
-  if (i < n && ss.active[i]) {
-    ss.geom_path[i] += hs.geom_step[i];
-    if (ss.left_world[i]) {
+  if (i >= 0) {
+    const double path = ss.geom_path[i];
+    ElState<R> el;
+    Rng rng;
+    StepLoop<R> L;
+    LoadSubstep(t, hs, ss, n, i, seed, el, L, rng);
+    ss.geom_path[i] = path + hs.geom_step[i];
+    if (L.left) {
       ss.active[i] = 0;
       ss.more[i] = 0;
     } else {
-      ElState<R> el;
-      Rng rng;
-      InitElectron(t, n, i, seed, el, rng);
-      LoadElectronHowFar(hs, n, i, el);
       el.preEkin = el.t.ekin;
       el.preLEkin = el.t.logE();
-      StepLoop<R> L;
-      LoadLoop(ss, i, L);
       const bool sampled = LoopAlong(T, el, L, rng);
       StoreElectronState(t, n, i, el, rng);
       t.ekin[i] = el.t.ekin;
@@ -243,39 +309,73 @@ __global__ void __launch_bounds__(kBlock) k_el_substep_along(DevTables<R> T, uin
   CountWave(&counters[4], again);
 }
 
+// Stage 2 of an e-/e+ slot: the final state of the chosen interaction
+// (PerformDiscrete, G4HepEmElectronManager.icc:443-458).
 template <typename R>
-__global__ void __launch_bounds__(kBlock) k_el_end(DevTables<R> T, uint64_t seed, hepem_tracks t, hepem_howfar_state hs,
-                                                   hepem_substep_state ss, hepem_step_out res) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  const int n = t.n;
-  if (i >= n) return;
-  const int8_t pt = t.ptype[i];
-  if ((pt != 0 && pt != 1) || hs.winner[i] == -99) {
-    WriteRejected<R>(t, t, res, n, i);
-    return;
-  }
-  ElState<R> el;
+HD void ElectronInteract(const DevTables<R>& T, uint64_t seed, hepem_tracks& out, const hepem_step_out& res, int n, int i,
+                         const Staged& r, uint8_t code) {
+  Trk<R> t;
   Rng rng;
-  InitElectron(t, n, i, seed, el, rng);
-  LoadElectronHowFar(hs, n, i, el);
-  StepLoop<R> L;
-  LoadLoop(ss, i, L);
+  Unstage(r, code, seed, t, rng);
   SecList<R> sl;
   sl.ns = 0;
-  LoopFinish(T, el, L, sl, rng);
-  StoreElectronState(t, n, i, el, rng);
-  t.ekin[i] = el.t.ekin;
+  ElectronFinal(T, t, code & kCodeProc, sl, rng);
+  out.ekin[i] = t.ekin;
 #pragma unroll
-  for (int c = 0; c < 3; ++c) t.dir[c * n + i] = (double)el.t.dir[c];
+  for (int c = 0; c < 3; ++c) out.dir[c * n + i] = (double)t.dir[c];
+  StoreRng(out, i, rng);
+  res.stopped[i] = t.ekin <= 0.0 ? 1 : 0;
+  WriteSecondaries(res, n, i, sl);
+}
+
+// The end of a slot's step up to its final state: the code of a pending one
+// (its record at st[j]), or 0.
+template <typename R>
+HD uint8_t EndStep(const DevTables<R>& T, uint64_t seed, hepem_tracks& t, const hepem_howfar_state& hs, hepem_substep_state& ss,
+                   const hepem_step_out& res, int n, int i, Staged* st, int j) {
+  ElState<R> el;
+  Rng rng;
+  StepLoop<R> L;
+  LoadSubstep(t, hs, ss, n, i, seed, el, L, rng);
+  const double path = ss.geom_path[i];
+  SecList<R> sl;
+  sl.ns = 0;
+  const uint8_t proc = ElectronProc(T, el.t, LoopFinishSelect(T, el, L, sl, rng));
+  StoreElectronState(t, n, i, el, rng);
   ss.stopped[i] = L.stopped ? 1 : 0;
   res.true_step[i] = (double)L.truePath;
-  res.geom_step[i] = ss.geom_path[i];
+  res.geom_step[i] = path;
   res.edep[i] = el.t.edep;
 #pragma unroll
   for (int c = 0; c < 3; ++c) res.displacement[c * n + i] = 0.0;
   res.winner[i] = el.t.winner;
+  if (proc != kPNone) {
+    const double d[3] = {(double)el.t.dir[0], (double)el.t.dir[1], (double)el.t.dir[2]};
+    return StageTrack(st, j, proc, el.t.isEl, el.t.imc, t.id[i], StreamHi(t, i), el.t.ekin, d, rng, 0.0);
+  }
+  t.ekin[i] = el.t.ekin;
+#pragma unroll
+  for (int c = 0; c < 3; ++c) t.dir[c * n + i] = (double)el.t.dir[c];
   res.stopped[i] = el.t.ekin <= 0.0 ? 1 : 0;
   WriteSecondaries(res, n, i, sl);
+  return kPNone;
+}
+
+template <typename R>
+__global__ void __launch_bounds__(kBlock) k_el_end(DevTables<R> T, uint64_t seed, hepem_tracks t, hepem_howfar_state hs,
+                                                   hepem_substep_state ss, hepem_step_out res) {
+  __shared__ BlockFinals<kBlock> fin;
+  const int i0 = blockIdx.x * kBlock, i = i0 + (int)threadIdx.x;
+  const int n = t.n;
+  uint8_t code = kPNone;
+  if (i < n) {
+    const int8_t pt = t.ptype[i];
+    if ((pt != 0 && pt != 1) || hs.winner[i] == -99) WriteRejected<R>(t, t, res, n, i);
+    else code = EndStep(T, seed, t, hs, ss, res, n, i, fin.st, (int)threadIdx.x);
+  }
+  SampleBlock<kBlock, kPIoniEl, kPAnnih>(fin, code, [&](int j, const Staged& r, uint8_t c, int) {
+    ElectronInteract<R>(T, seed, t, res, n, i0 + j, r, c);
+  });
 }
 
 // ---- two-stage step: particle sort, then process sort ----------------------------------------
@@ -446,25 +546,6 @@ HD uint8_t PerformGammaSelect(const DevTables<R>& T, uint64_t seed, hepem_tracks
   Rng rng;
   rng.init(seed, (uint32_t)t.id[i], StreamHi(t, i), t.rng_ctr[i], t.rng_has_gauss[i] != 0, t.rng_gauss[i]);
   return GammaSelectAfterHowFar(T, g, (R)hs.pe_xsec[i], rng, t, t, res, st, n, i);
-}
-
-// Stage 2 of an e-/e+ slot: the final state of the chosen interaction
-// (PerformDiscrete, G4HepEmElectronManager.icc:443-458).
-template <typename R>
-HD void ElectronInteract(const DevTables<R>& T, uint64_t seed, hepem_tracks& out, const hepem_step_out& res, int n, int i,
-                         const Staged& r, uint8_t code) {
-  Trk<R> t;
-  Rng rng;
-  Unstage(r, code, seed, t, rng);
-  SecList<R> sl;
-  sl.ns = 0;
-  ElectronFinal(T, t, code & kCodeProc, sl, rng);
-  out.ekin[i] = t.ekin;
-#pragma unroll
-  for (int c = 0; c < 3; ++c) out.dir[c * n + i] = (double)t.dir[c];
-  StoreRng(out, i, rng);
-  res.stopped[i] = t.ekin <= 0.0 ? 1 : 0;
-  WriteSecondaries(res, n, i, sl);
 }
 
 // Stage 2 of a gamma slot: the interaction and the gamma tracking cut of
