@@ -26,6 +26,18 @@ constexpr double kALargeValue = 1.0E+20;
 constexpr int kPoissonMaxTerms = 1000;
 constexpr int kSBGuide = 32;           // buckets of the SB search guide
 
+// The arguments of a kernel that takes one struct A, to be read where they are
+// used: each call gives an address that the compiler cannot tell from another's,
+// so no argument read before it is held in scalar registers (or spilled from
+// them) past it.
+template <typename A> HD const A& KernelArgs() {
+  auto p = __builtin_amdgcn_kernarg_segment_ptr();
+#if defined(__HIP_DEVICE_COMPILE__)
+  asm volatile("" : "+s"(p));
+#endif
+  return *(const A*)p;
+}
+
 template <typename T> HD T tmax(T a, T b) { return a > b ? a : b; }
 template <typename T> HD T tmin(T a, T b) { return a < b ? a : b; }
 

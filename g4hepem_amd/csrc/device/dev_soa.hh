@@ -90,7 +90,7 @@ HD void CopyIdentity(const hepem_tracks& in, hepem_tracks& out, int i) {
   out.on_boundary[i] = in.on_boundary[i];
 }
 
-HD void StoreRng(hepem_tracks& out, int i, const Rng& rng) {
+HD void StoreRng(const hepem_tracks& out, int i, const Rng& rng) {
   out.rng_ctr[i] = rng.ctr;
   out.rng_gauss[i] = rng.gauss;
   out.rng_has_gauss[i] = rng.has_gauss ? 1 : 0;

@@ -635,6 +635,16 @@ extern "C" int hepem_step_prepare(const hepem_ctx* c, const hepem_tracks* in, vo
   return PrepareQueue(c, in, work, stream, SortsProcesses(c));
 }
 
+namespace {
+// The step in one launch (k_step_block) instead of two stages: always in the
+// FP32-table form; in FP64 up to the slots of one resident round of its blocks
+// (256 CUs x 3 blocks): to there it is faster in both orders of the slots (131k
+// mixed 66 us against 75, 200k ordered 79 against 98), and beyond, where a
+// second round begins, slower (262k mixed 111 against 100).
+constexpr int kBlockStepMax64 = 256 * 3 * kBlock;
+bool StepsInOneLaunch(const hepem_ctx* c, int n) { return c->precision != HEPEM_FP64 || n <= kBlockStepMax64; }
+}  // namespace
+
 extern "C" int hepem_step_run(const hepem_ctx* c, uint64_t seed, const hepem_tracks* in, hepem_tracks* out,
                               hepem_step_out* res, void* work, void* stream) {
   if (!c || !TracksOk(in) || !TracksOk(out) || !ResOk(res, in->n) || out->n != in->n || !work) return HEPEM_ERR_INVALID;
@@ -651,22 +661,20 @@ extern "C" int hepem_step_run(const hepem_ctx* c, uint64_t seed, const hepem_tra
     else
       hipLaunchKernelGGL(k_step<float>, dim3(grid), dim3(kBlock), 0, s, c->t32, seed, *in, *out, *res, w.queue, w.counters,
                          w.tinfo);
+  } else if (StepsInOneLaunch(c, n)) {
+    if (fp64)
+      hipLaunchKernelGGL(k_step_block<double>, dim3(LocalSelectGrid(n)), dim3(kBlock), 0, s,
+                         StepArgs<double>{c->t64, seed, *in, *out, *res, w.queue, w.counters, w.tinfo, w.code, w.st});
+    else
+      hipLaunchKernelGGL(k_step_block<float>, dim3(LocalSelectGrid(n)), dim3(kBlock), 0, s,
+                         StepArgs<float>{c->t32, seed, *in, *out, *res, w.queue, w.counters, w.tinfo, w.code, w.st});
   } else {
     const int tiles = (n + kClassifyTile - 1) / kClassifyTile;
-    const int igrid = InteractGrid(n);
-    if (fp64) {
-      hipLaunchKernelGGL(k_step_select_local<double>, dim3(LocalSelectGrid(n)), dim3(kBlock), 0, s, c->t64, seed, *in, *out, *res, w.queue,
-                         w.counters, w.tinfo, w.code, w.st);
-      hipLaunchKernelGGL(k_classify_tiles, dim3(tiles), dim3(kClassifyBlock), 0, s, n, w.code, w.tlist, w.tinfo);
-      hipLaunchKernelGGL(k_interact_tiles<double>, dim3(igrid), dim3(kBlock), 0, s, c->t64, seed, *out, *res, w.code, w.st,
-                         w.tlist, w.tinfo);
-    } else {
-      hipLaunchKernelGGL(k_step_select_local<float>, dim3(LocalSelectGrid(n)), dim3(kBlock), 0, s, c->t32, seed, *in, *out, *res, w.queue,
-                         w.counters, w.tinfo, w.code, w.st);
-      hipLaunchKernelGGL(k_classify_tiles, dim3(tiles), dim3(kClassifyBlock), 0, s, n, w.code, w.tlist, w.tinfo);
-      hipLaunchKernelGGL(k_interact_tiles<float>, dim3(igrid), dim3(kBlock), 0, s, c->t32, seed, *out, *res, w.code, w.st,
-                         w.tlist, w.tinfo);
-    }
+    hipLaunchKernelGGL(k_step_select_local<double>, dim3(LocalSelectGrid(n)), dim3(kBlock), 0, s,
+                       StepArgs<double>{c->t64, seed, *in, *out, *res, w.queue, w.counters, w.tinfo, w.code, w.st});
+    hipLaunchKernelGGL(k_classify_tiles, dim3(tiles), dim3(kClassifyBlock), 0, s, n, w.code, w.tlist, w.tinfo);
+    hipLaunchKernelGGL(k_interact_tiles<double>, dim3(InteractGrid(n)), dim3(kBlock), 0, s, c->t64, seed, *out, *res, w.code, w.st,
+                       w.tlist, w.tinfo);
   }
   HIP_OK(hipGetLastError());
   return HEPEM_OK;

@@ -379,6 +379,8 @@ __global__ void __launch_bounds__(kBlock) k_el_end(DevTables<R> T, uint64_t seed
 }
 
 // ---- two-stage step: particle sort, then process sort ----------------------------------------
+// (the FP32-table form and the smaller FP64 batches take the step in one launch
+// instead: k_step_block)
 // k_step_select_local does HowFar, the continuous step and the choice of the
 // discrete interaction (one thread per particle-queue entry), records the chosen process
 // per slot and, for a pending interaction, the 64-byte record of what the
@@ -392,7 +394,7 @@ __global__ void __launch_bounds__(kBlock) k_el_end(DevTables<R> T, uint64_t seed
 // PerformDiscrete's choice (G4HepEmElectronManager.icc:425-441,461-483).
 // Returns the slot code; a complete step (kPNone) also gets its post-step
 // kinematics, secondaries and stopped flag here, a pending one its staged
-// record.
+// record at st[j].
 //
 // Every field is stored as soon as it is final, not at the end: the MSC state,
 // the interaction lengths and the mean free paths would otherwise hold about 30
@@ -404,7 +406,7 @@ __global__ void __launch_bounds__(kBlock) k_el_end(DevTables<R> T, uint64_t seed
 // 162 instead of 169, 1M mixed tracks 314 instead of 318.
 template <typename R>
 HD uint8_t ElectronSelectAfterHowFar(const DevTables<R>& T, ElState<R>& el, Rng& rng, const hepem_tracks& in,
-                                     hepem_tracks& out, const hepem_step_out& res, Staged* st, int n, int i) {
+                                     hepem_tracks& out, const hepem_step_out& res, int n, int i, Staged* st, int j) {
   Trk<R>& t = el.t;
   const int winner = t.winner;
   {
@@ -447,7 +449,7 @@ HD uint8_t ElectronSelectAfterHowFar(const DevTables<R>& T, ElState<R>& el, Rng&
   }
   if (proc != kPNone) {
     const double d[3] = {(double)t.dir[0], (double)t.dir[1], (double)t.dir[2]};
-    return StageTrack(st, i, proc, t.isEl, t.imc, in.id[i], StreamHi(in, i), t.ekin, d, rng, 0.0);
+    return StageTrack(st, j, proc, t.isEl, t.imc, in.id[i], StreamHi(in, i), t.ekin, d, rng, 0.0);
   }
   out.ekin[i] = t.ekin;
 #pragma unroll
@@ -467,7 +469,7 @@ HD uint8_t PerformElectronSelect(const DevTables<R>& T, uint64_t seed, hepem_tra
   Rng rng;
   InitElectron(t, n, i, seed, el, rng);
   LoadElectronHowFar(hs, n, i, el);
-  return ElectronSelectAfterHowFar(T, el, rng, t, t, res, st, n, i);
+  return ElectronSelectAfterHowFar(T, el, rng, t, t, res, n, i, st, i);
 }
 
 // Stage 1 of a gamma slot after its HowFar: SelectInteraction and the
@@ -475,7 +477,7 @@ HD uint8_t PerformElectronSelect(const DevTables<R>& T, uint64_t seed, hepem_tra
 // (G4HepEmGammaManager.icc:54-62,173-219; G4HepEmTrackingManager.cc:1092-1108).
 template <typename R>
 HD uint8_t GammaSelectAfterHowFar(const DevTables<R>& T, Trk<R>& t, R pe, Rng& rng, const hepem_tracks& in,
-                                  hepem_tracks& out, const hepem_step_out& res, Staged* st, int n, int i) {
+                                  hepem_tracks& out, const hepem_step_out& res, int n, int i, Staged* st, int j) {
   const uint8_t proc = GammaProc(T, t, pe, rng);
 #pragma unroll
   for (int k = 0; k < 4; ++k) out.num_ia_left[k * n + i] = (double)t.nial[k];
@@ -486,7 +488,7 @@ HD uint8_t GammaSelectAfterHowFar(const DevTables<R>& T, Trk<R>& t, R pe, Rng& r
   res.winner[i] = t.winner;
   if (proc != kPNone) {
     const double d[3] = {(double)t.dir[0], (double)t.dir[1], (double)t.dir[2]};
-    return StageTrack(st, i, proc, false, t.imc, in.id[i], StreamHi(in, i), t.ekin, d, rng, (double)pe);
+    return StageTrack(st, j, proc, false, t.imc, in.id[i], StreamHi(in, i), t.ekin, d, rng, (double)pe);
   }
   out.ekin[i] = t.ekin;
 #pragma unroll
@@ -500,37 +502,47 @@ HD uint8_t GammaSelectAfterHowFar(const DevTables<R>& T, Trk<R>& t, R pe, Rng& r
   return kPNone;
 }
 
+// What stage 1 of the step works on.
+template <typename R> struct StepView {
+  const DevTables<R>& T;
+  uint64_t seed;
+  const hepem_tracks& in;
+  hepem_tracks& out;
+  const hepem_step_out& res;
+  uint32_t* counters;
+};
+
 // Stage 1 of slot i of the step: its whole state loaded at once, the test of
-// its couple and energy, the identity copy, HowFar and the selection. Records
-// the slot's code.
-template <typename R>
-HD void StepSelect(const DevTables<R>& T, uint64_t seed, const hepem_tracks& in, hepem_tracks& out, const hepem_step_out& res,
-                   uint32_t* counters, uint8_t* code, Staged* st, int n, int i, bool isE) {
-  TrackIn r = LoadTrackIn(in, n, i);
+// its couple and energy, the identity copy, HowFar and the selection. Returns
+// the slot's code; a pending slot's record goes to st[j]. view() gives the
+// StepView; it is asked for again after HowFar.
+template <typename R, typename V> HD uint8_t StepSelect(V view, int n, int i, bool isE, Staged* st, int j) {
+  const StepView<R> v = view();
+  TrackIn r = LoadTrackIn(v.in, n, i);
   MscIn q{};
-  if (isE) q = LoadMscIn(in, i);
+  if (isE) q = LoadMscIn(v.in, i);
   KeepLoaded(r);
-  if (!TrackValid(T, r.imc, r.ekin)) {
-    atomicAdd(&counters[2], 1u);
-    WriteRejected<R>(in, out, res, n, i);
-    code[i] = kPNone;
-    return;
+  if (!TrackValid(v.T, r.imc, r.ekin)) {
+    atomicAdd(&v.counters[2], 1u);
+    WriteRejected<R>(v.in, v.out, v.res, n, i);
+    return kPNone;
   }
-  StoreIdentity(in, out, i, r);
+  StoreIdentity(v.in, v.out, i, r);
   Rng rng;
   if (isE) {
     ElState<R> el;
-    InitElectron(r, q, seed, el, rng);
-    ElectronHowFar(T, el, rng);
-    code[i] = ElectronSelectAfterHowFar(T, el, rng, in, out, res, st, n, i);
-  } else {
-    Trk<R> t;
-    t.isEl = false;
-    InitTrack(r, t);
-    InitRng(r, seed, rng);
-    const R pe = GammaHowFar(T, t, rng);
-    code[i] = GammaSelectAfterHowFar(T, t, pe, rng, in, out, res, st, n, i);
+    InitElectron(r, q, v.seed, el, rng);
+    ElectronHowFar(v.T, el, rng);
+    const StepView<R> w = view();
+    return ElectronSelectAfterHowFar(w.T, el, rng, w.in, w.out, w.res, n, i, st, j);
   }
+  Trk<R> t;
+  t.isEl = false;
+  InitTrack(r, t);
+  InitRng(r, v.seed, rng);
+  const R pe = GammaHowFar(v.T, t, rng);
+  const StepView<R> w = view();
+  return GammaSelectAfterHowFar(w.T, t, pe, rng, w.in, w.out, w.res, n, i, st, j);
 }
 
 // Stage 1 of a gamma slot of the split Perform: step, mean free path and PE
@@ -545,7 +557,7 @@ HD uint8_t PerformGammaSelect(const DevTables<R>& T, uint64_t seed, hepem_tracks
   g.mfp[0] = (R)hs.mfp[i];
   Rng rng;
   rng.init(seed, (uint32_t)t.id[i], StreamHi(t, i), t.rng_ctr[i], t.rng_has_gauss[i] != 0, t.rng_gauss[i]);
-  return GammaSelectAfterHowFar(T, g, (R)hs.pe_xsec[i], rng, t, t, res, st, n, i);
+  return GammaSelectAfterHowFar(T, g, (R)hs.pe_xsec[i], rng, t, t, res, n, i, st, i);
 }
 
 // Stage 2 of a gamma slot: the interaction and the gamma tracking cut of
@@ -694,26 +706,88 @@ __device__ inline bool LocalSelectChunk(int ntiles, int& tile, int& chunk) {
   return true;
 }
 
+// The arguments of the step's kernels.
+template <typename R> struct StepArgs {
+  DevTables<R> T;
+  uint64_t seed;
+  hepem_tracks in, out;
+  hepem_step_out res;
+  const uint32_t* queue;
+  uint32_t* counters;
+  const uint32_t* tinfo;
+  uint8_t* code;   // of the two-stage step
+  Staged* st;
+};
+// The StepView of a kernel that takes one StepArgs. Read anew after HowFar, the
+// arguments leave k_step_select_local 125 VGPRs and no spills (128 and 10 with
+// them held: 1M tracks 288 us instead of 294, 3M ordered 681 instead of 699) and
+// the FP32-table form of k_step_block 97 instead of 119.
+template <typename R> HD StepView<R> ArgsView() {
+  const StepArgs<R>& a = KernelArgs<StepArgs<R>>();
+  return {a.T, a.seed, a.in, const_cast<hepem_tracks&>(a.out), a.res, a.counters};
+}
+// The slot of this thread in a grid of LocalSelectGrid(n) blocks and whether it
+// holds an e-/e+, in the layout hepem_step_prepare chose (tile-local, or e-/e+
+// first over the batch); -1 without a slot. `none`: so is the whole block.
+template <typename R> __device__ __forceinline__ int StepSlot(bool& isE, bool& none) {
+  const StepArgs<R>& a = KernelArgs<StepArgs<R>>();
+  const int n = a.in.n;
+  int tile, chunk;
+  none = true;
+  if (!LocalSelectChunk((n + kClassifyTile - 1) / kClassifyTile, tile, chunk)) return -1;
+  const int tile0 = tile * kClassifyTile;
+  const int m = min(kClassifyTile, n - tile0);
+  none = chunk * kBlock >= m;
+  const int jl = chunk * kBlock + (int)threadIdx.x;
+  if (jl >= m) return -1;
+  isE = a.counters[kCounterLayout] ? jl < (int)a.tinfo[(size_t)tile * kTileInfo] : (uint32_t)(tile0 + jl) < a.counters[0];
+  return (int)a.queue[tile0 + jl];
+}
+
 // Stage 1 of the step over one batch's particle queue, its blocks placed tile by
 // tile as LocalSelectChunk places them (the tile-local partition that
 // hepem_step_prepare lays out with the process sort; a queue laid out over the
 // whole batch is read correctly too).
+template <typename R> __global__ void __launch_bounds__(kBlock, 4) k_step_select_local(StepArgs<R>) {
+  bool isE = false, none;
+  const int i = StepSlot<R>(isE, none);
+  if (i < 0) return;
+  const uint8_t c = StepSelect<R>([] { return ArgsView<R>(); }, KernelArgs<StepArgs<R>>().in.n, i, isE,
+                                  KernelArgs<StepArgs<R>>().st, i);
+  KernelArgs<StepArgs<R>>().code[i] = c;
+}
+
+// The whole step in one launch: stage 1 as k_step_select_local, then the final
+// states of the block's pending slots, sorted by process within the block.
+//
+// Bound by the latency of one wave's chain in a small batch, by VALU issue in a
+// large one. Against the three launches of the two-stage step it keeps the
+// pending state in LDS instead of 130 bytes a slot through memory and runs the
+// chain of a track in one go; the two-stage step fills the waves of the final
+// states better and, in FP64, has 4 waves per SIMD (this kernel 3: held to 4 it
+// spills and 1M tracks take 320 us). The FP32-table form runs 5 waves per SIMD
+// (4 VGPRs spilled; left alone it takes 97 VGPRs, 4 waves, and 1M tracks 243 us)
+// and is faster at every size: 16k ordered tracks 44.5 us instead of 50, 1M
+// mixed 225 instead of 260, 3M 588 instead of 756. FP64: 131k 67 instead of 76,
+// 200k 92 and 92, 300k 117 and 108, 1M 309 and 294.
+template <typename R> constexpr int kStepBlockWaves = sizeof(R) == sizeof(double) ? 3 : 5;
 template <typename R>
-__global__ void __launch_bounds__(kBlock, 4) k_step_select_local(DevTables<R> T, uint64_t seed, hepem_tracks in, hepem_tracks out,
-                                                        hepem_step_out res, const uint32_t* __restrict__ queue,
-                                                        uint32_t* __restrict__ counters, const uint32_t* __restrict__ tinfo,
-                                                        uint8_t* __restrict__ code, Staged* __restrict__ st) {
-  const int n = in.n;
-  int tile, chunk;
-  if (!LocalSelectChunk((n + kClassifyTile - 1) / kClassifyTile, tile, chunk)) return;
-  const int tile0 = tile * kClassifyTile;
-  const int m = min(kClassifyTile, n - tile0);
-  const int jl = chunk * kBlock + (int)threadIdx.x;
-  if (jl >= m) return;
-  // the layout hepem_step_prepare chose: tile-local, or e-/e+ first over the batch
-  const bool isE = counters[kCounterLayout] ? jl < (int)tinfo[(size_t)tile * kTileInfo] : (uint32_t)(tile0 + jl) < counters[0];
-  const int i = (int)queue[tile0 + jl];
-  StepSelect(T, seed, in, out, res, counters, code, st, n, i, isE);
+__global__ void __launch_bounds__(kBlock, kStepBlockWaves<R>) k_step_block(StepArgs<R>) {
+  __shared__ BlockFinals<kBlock> fin;
+  __shared__ int32_t slot[kBlock];
+  uint8_t code = kPNone;
+  bool isE = false, none;
+  const int i = StepSlot<R>(isE, none);
+  if (none) return;  // the whole block
+  slot[threadIdx.x] = i;
+  if (i >= 0)
+    code = StepSelect<R>([] { return ArgsView<R>(); }, KernelArgs<StepArgs<R>>().in.n, i, isE, fin.st, (int)threadIdx.x);
+  SampleBlock<kBlock, kPIoniEl, kPPE>(fin, code, [&](int j, const Staged& r, uint8_t c, int proc) {
+    const StepArgs<R>& a = KernelArgs<StepArgs<R>>();
+    hepem_tracks& out = const_cast<hepem_tracks&>(a.out);
+    if (proc < kPConv) ElectronInteract<R>(a.T, a.seed, out, a.res, a.in.n, slot[j], r, c);
+    else GammaInteract<R>(a.T, a.seed, out, a.res, a.in.n, slot[j], r, c);
+  });
 }
 
 // Thread -> (slot, is-e-/e+) of the split HowFar and Perform kernels. A
@@ -1095,7 +1169,7 @@ __device__ void StepSelectChunk(const DevTables<R>& T, uint64_t seed, const Batc
   uint32_t* cnt = bcounters + 4 * b;
   const uint32_t qoff = d[b].qoff;
   const int i = (int)queue[qoff + j];
-  StepSelect(T, seed, in, out, res, cnt, code + qoff, st + qoff, n, i, (uint32_t)j < cnt[0]);
+  code[qoff + i] = StepSelect<R>([&] { return StepView<R>{T, seed, in, out, res, cnt}; }, n, i, (uint32_t)j < cnt[0], st + qoff, i);
 }
 
 // The tile-local particle partition over every batch: block t lays out
@@ -1136,7 +1210,8 @@ __global__ void __launch_bounds__(kBlock, 4) k_step_select_local_batched(DevTabl
   if (jl >= m) return;
   const uint32_t qoff = d[b].qoff;
   const int i = (int)queue[qoff + tile0 + jl];
-  StepSelect(T, seed, in, out, res, bcounters + 4 * b, code + qoff, st + qoff, n, i, jl < (int)ecount[tile]);
+  code[qoff + i] = StepSelect<R>([&] { return StepView<R>{T, seed, in, out, res, bcounters + 4 * b}; }, n, i, jl < (int)ecount[tile],
+                                 st + qoff, i);
 }
 
 // Next work item of a persistent kernel: thread 0 takes it from *next and the
