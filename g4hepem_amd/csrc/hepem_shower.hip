@@ -292,7 +292,7 @@ __device__ bool WoodcockStep(const hepem::DevTables<R>& T, const Slabs& g, hepem
 // end of the round needs of it (its energy, the deposit, the secondaries' number,
 // kinds and energies).
 template <typename R>
-__device__ __forceinline__ void StoreFinal(hepem_tracks& t, const hepem_step_out& res, int n, int i, const hepem::Trk<R>& k,
+__device__ __forceinline__ void StoreFinal(const hepem_tracks& t, const hepem_step_out& res, int n, int i, const hepem::Trk<R>& k,
                                            const hepem::Rng& rng, const hepem::SecList<R>& sl, double edep, hepem::Staged& r) {
   t.ekin[i] = k.ekin;
 #pragma unroll
@@ -312,6 +312,19 @@ __device__ __forceinline__ void StoreFinal(hepem_tracks& t, const hepem_step_out
     r.stream = (uint32_t)sl.s1.ptype;
   }
 }
+// The arguments of the stepping kernel.
+template <typename R> struct MoveArgs {
+  Stack s;
+  Slabs g;
+  hepem_step_out res;
+  hepem::DevTables<R> T;
+  uint64_t seed;
+  int ne, ge;
+  unsigned long long *dep, *leak;
+  uint8_t* next;
+  uint32_t *offE, *offG, *bsumE, *bsumG, *bsec;
+};
+
 // Where a slot's move ended, held by its thread to the end of the round.
 struct Moved {
   double x;      // position
@@ -333,50 +346,58 @@ struct Moved {
 // an interaction whose final state is pending, with its record at st[j] (and the
 // step's deposit in its pe), or 0.
 template <typename R>
-__device__ __forceinline__ uint8_t ElectronSubstep(const Stack& s, const Slabs& g, const hepem_step_out& res,
-                                                   const hepem::DevTables<R>& T, uint64_t seed, int i, Moved& mv,
-                                                   hepem::Staged* st, int j) {
+__device__ __forceinline__ uint8_t ElectronSubstep(int n, int i, Moved& mv, hepem::Staged* st, int j) {
   using namespace hepem;
-  const int n = s.t.n;
-  hepem_tracks t = s.t;
-  const int l = s.layer[i];
   ElState<R> el;
   Rng rng;
-  TrackIn in = LoadTrackIn(t, n, i);
-  const MscIn q = LoadMscIn(t, i);
-  KeepLoaded(in);
-  InitElectron(in, q, seed, el, rng);
   StepLoop<R> L;
-  SlabPos p{s.x[i], g.plane[l], g.plane[l + 1], l == 0, l == g.nbins - 1, 0};
-  const uint8_t f0 = s.lp.flags[i];
-  if (!(f0 & kInStep)) {
-    SlabBegin(T, el, L, rng, p);
-    t.safety[i] = (double)el.t.safety;
-    s.lp.preEkin[i] = L.preEkin;
-    s.lp.iDProc[i] = (int8_t)L.iDProc;
+  SlabPos p;
+  int l;
+  TrackIn in;
+  {
+    const MoveArgs<R>& a = KernelArgs<MoveArgs<R>>();
+    const Stack& s = a.s;
+    const Slabs& g = a.g;
+    const hepem_tracks& t = s.t;
+    l = s.layer[i];
+    in = LoadTrackIn(t, n, i);
+    const MscIn q = LoadMscIn(t, i);
+    KeepLoaded(in);
+    InitElectron(in, q, a.seed, el, rng);
+    p = SlabPos{s.x[i], g.plane[l], g.plane[l + 1], l == 0, l == g.nbins - 1, 0};
+    const uint8_t f0 = s.lp.flags[i];
+    if (!(f0 & kInStep)) {
+      SlabBegin(a.T, el, L, rng, p);
+      t.safety[i] = (double)el.t.safety;
+      s.lp.preEkin[i] = L.preEkin;
+      s.lp.iDProc[i] = (int8_t)L.iDProc;
 #pragma unroll
-    for (int k = 0; k < 4; ++k) s.lp.mfp[k * n + i] = (double)el.t.mfp[k];
-  } else {
+      for (int k = 0; k < 4; ++k) s.lp.mfp[k * n + i] = (double)el.t.mfp[k];
+    } else {
 #pragma unroll
-    for (int k = 0; k < 4; ++k) el.t.mfp[k] = (R)s.lp.mfp[k * n + i];
-    el.range = (R)s.lp.range[i];
-    el.pstep = (R)s.lp.stepLeft[i];
-    el.t.gstep = el.pstep;  // HowFarToMSC keeps it where MSC is off
-    el.preEkin = el.t.ekin;
-    el.preLEkin = el.t.logE();
-    L.iDProc = s.lp.iDProc[i];
-    el.t.winner = L.iDProc;
-    L.stepLeft = el.pstep;
-    L.truePath = (R)0.;
-    L.meanLoss = s.lp.meanLoss[i];
-    L.preEkin = s.lp.preEkin[i];
-    L.preLEkin = (R)0.;
-    L.cont = (f0 & kCont) != 0;
-    L.stopped = false;
-    L.left = false;
-    L.nsub = s.lp.nsub[i];
+      for (int k = 0; k < 4; ++k) el.t.mfp[k] = (R)s.lp.mfp[k * n + i];
+      el.range = (R)s.lp.range[i];
+      el.pstep = (R)s.lp.stepLeft[i];
+      el.t.gstep = el.pstep;  // HowFarToMSC keeps it where MSC is off
+      el.preEkin = el.t.ekin;
+      el.preLEkin = el.t.logE();
+      L.iDProc = s.lp.iDProc[i];
+      el.t.winner = L.iDProc;
+      L.stepLeft = el.pstep;
+      L.truePath = (R)0.;
+      L.meanLoss = s.lp.meanLoss[i];
+      L.preEkin = s.lp.preEkin[i];
+      L.preLEkin = (R)0.;
+      L.cont = (f0 & kCont) != 0;
+      L.stopped = false;
+      L.left = false;
+      L.nsub = s.lp.nsub[i];
+    }
   }
-  const bool done = SlabSubstep(T, el, L, rng, p);
+  const bool done = SlabSubstep(KernelArgs<MoveArgs<R>>().T, el, L, rng, p);
+  const MoveArgs<R>& a = KernelArgs<MoveArgs<R>>();
+  const Stack& s = a.s;
+  const hepem_tracks& t = s.t;
   const R rangeLeft = el.range;
   t.on_boundary[i] = p.side != 0 ? 1 : 0;
   mv.x = p.x;
@@ -397,7 +418,7 @@ __device__ __forceinline__ uint8_t ElectronSubstep(const Stack& s, const Slabs& 
   if (done) {
     L.preLEkin = L.preEkin > 0. ? vlog((R)L.preEkin) : (R)-30;
     s.lp.flags[i] = 0;
-    proc = ElectronProc(T, el.t, LoopFinishSelect(T, el, L, sl, rng));
+    proc = ElectronProc(a.T, el.t, LoopFinishSelect(a.T, el, L, sl, rng));
     edep = el.t.edep;
   } else {
     s.lp.range[i] = (double)rangeLeft;
@@ -412,7 +433,7 @@ __device__ __forceinline__ uint8_t ElectronSubstep(const Stack& s, const Slabs& 
     const double d[3] = {(double)el.t.dir[0], (double)el.t.dir[1], (double)el.t.dir[2]};
     return StageTrack(st, j, proc, el.t.isEl, el.t.imc, in.id, in.stream, el.t.ekin, d, rng, edep);
   }
-  StoreFinal(t, res, n, i, el.t, rng, sl, edep, st[j]);
+  StoreFinal(t, a.res, n, i, el.t, rng, sl, edep, st[j]);
   return kPNone;
 }
 
@@ -423,12 +444,12 @@ __device__ __forceinline__ uint8_t ElectronSubstep(const Stack& s, const Slabs& 
 // SelectInteraction. The pending interaction as ElectronSubstep's (pe = the PE
 // cross section); the slab of the deposit is changed only by a Woodcock step.
 template <typename R, bool kWoodcock>
-__device__ __forceinline__ uint8_t GammaStep(const Stack& s, const Slabs& g, const hepem_step_out& res,
-                                             const hepem::DevTables<R>& T, uint64_t seed, int i, Moved& mv, hepem::Staged* st,
-                                             int j) {
+__device__ __forceinline__ uint8_t GammaStep(int n, int i, Moved& mv, hepem::Staged* st, int j) {
   using namespace hepem;
-  const int n = s.t.n;
-  hepem_tracks t = s.t;
+  const MoveArgs<R>& a = KernelArgs<MoveArgs<R>>();
+  const Stack& s = a.s;
+  const Slabs& g = a.g;
+  const hepem_tracks& t = s.t;
   int l = s.layer[i];
   const double x = s.x[i];
   Trk<R> gt;
@@ -437,12 +458,12 @@ __device__ __forceinline__ uint8_t GammaStep(const Stack& s, const Slabs& g, con
   KeepLoaded(in);
   InitTrack(in, gt);
   Rng rng;
-  InitRng(in, seed, rng);
-  R pe = GammaHowFar(T, gt, rng);
+  InitRng(in, a.seed, rng);
+  R pe = GammaHowFar(a.T, gt, rng);
   const double ux = (double)gt.dir[0];
   double xe;
   int sd = 0;
-  if (!(kWoodcock && gt.ekin > g.wdtMin && WoodcockStep(T, g, gt, rng, pe, l, x, ux, xe, sd))) {
+  if (!(kWoodcock && gt.ekin > g.wdtMin && WoodcockStep(a.T, g, gt, rng, pe, l, x, ux, xe, sd))) {
     const double gs = (double)gt.gstep;
     double dist = 1.0e300;
     if (ux > 0.0) {
@@ -465,7 +486,7 @@ __device__ __forceinline__ uint8_t GammaStep(const Stack& s, const Slabs& g, con
     s.layer[i] = l;
     t.imc[i] = gt.imc;
   }
-  const uint8_t proc = GammaProc(T, gt, pe, rng);
+  const uint8_t proc = GammaProc(a.T, gt, pe, rng);
   t.num_ia_left[i] = (double)gt.nial[0];
   t.on_boundary[i] = gt.onBoundary ? 1 : 0;
   mv.x = xe;
@@ -478,7 +499,7 @@ __device__ __forceinline__ uint8_t GammaStep(const Stack& s, const Slabs& g, con
   }
   SecList<R> sl;
   sl.ns = 0;
-  StoreFinal(t, res, n, i, gt, rng, sl, 0.0, st[j]);
+  StoreFinal(t, a.res, n, i, gt, rng, sl, 0.0, st[j]);
   return kPNone;
 }
 
@@ -504,8 +525,10 @@ __device__ __forceinline__ int BlockSlots(int n, int ne, int ge, int& i0) {
 // of its own read back ten arrays that this one had just written) takes the
 // position from registers and the rest from LDS. 1000 showers: 38.1 ms with the
 // sorted final states instead of 38.7, 35.1 instead of 36.5 without the kernel
-// that ended the round. Held to 3 waves per SIMD in FP64, 4 in the FP32-table
-// form.
+// that ended the round. The arguments are read anew at each stage (MoveArgs): held
+// to the end they spilled from scalar registers into VGPR lanes; 33.0 ms became
+// 32.1, in the FP32-table form 28.0 became 26.7 (168 -> 153 VGPRs, 128 -> 99).
+// Held to 3 waves per SIMD in FP64, 4 in the FP32-table form.
 //
 // End of the round. The next stack holds the e-/e+ first and the gammas after
 // them, each part in slot order of the parents. next[i]: bit s = secondary slot
@@ -519,9 +542,7 @@ constexpr uint8_t kSurvives = 4;
 constexpr int kHash = 2 * kB;
 template <typename R, bool kWoodcock>
 __global__ void __launch_bounds__(kB, sizeof(R) == sizeof(double) ? 3 : 4)
-    k_sh_move(Stack s, Slabs g, hepem_step_out res, hepem::DevTables<R> T, uint64_t seed, int ne, int ge, unsigned long long* dep,
-              unsigned long long* leak, uint8_t* __restrict__ next, uint32_t* __restrict__ offE, uint32_t* __restrict__ offG,
-              uint32_t* __restrict__ bsumE, uint32_t* __restrict__ bsumG, uint32_t* __restrict__ bsec) {
+    k_sh_move(MoveArgs<R>) {
   using namespace hepem;
   __shared__ union {
     BlockFinals<kB> fin;
@@ -529,38 +550,50 @@ __global__ void __launch_bounds__(kB, sizeof(R) == sizeof(double) ? 3 : 4)
       unsigned long long key[kHash], val[kHash];
     } hash;
   } sh;
-  const int n = s.t.n;
-  hepem_tracks t = s.t;
-  int i0;
-  const int last = BlockSlots(n, ne, ge, i0), i = i0 + (int)threadIdx.x;
-  const bool valid = i < last, isE = (int)blockIdx.x < ge;
+  int i0, last;
+  bool isE;
   uint8_t code = kPNone;
   Moved mv;
+  {
+    const MoveArgs<R>& a = KernelArgs<MoveArgs<R>>();
+    last = BlockSlots(a.s.t.n, a.ne, a.ge, i0);
+    isE = (int)blockIdx.x < a.ge;
+  }
+  const int i = i0 + (int)threadIdx.x;
+  const bool valid = i < last;
   if (isE) {
-    if (valid) code = ElectronSubstep(s, g, res, T, seed, i, mv, sh.fin.st, (int)threadIdx.x);
+    if (valid) code = ElectronSubstep<R>(KernelArgs<MoveArgs<R>>().s.t.n, i, mv, sh.fin.st, (int)threadIdx.x);
     SampleBlock<kB, kPIoniEl, kPAnnih>(sh.fin, code, [&](int j, Staged& r, uint8_t c, int proc) {
+      const MoveArgs<R>& a = KernelArgs<MoveArgs<R>>();
       Trk<R> k;
       Rng rng;
       SecList<R> sl;
       sl.ns = 0;
       const double edep = r.pe;
-      Unstage(r, c, seed, k, rng);
-      ElectronFinal(T, k, proc, sl, rng);
-      StoreFinal(t, res, n, i0 + j, k, rng, sl, edep, r);
+      Unstage(r, c, a.seed, k, rng);
+      ElectronFinal(a.T, k, proc, sl, rng);
+      const MoveArgs<R>& w = KernelArgs<MoveArgs<R>>();
+      StoreFinal(w.s.t, w.res, w.s.t.n, i0 + j, k, rng, sl, edep, r);
     });
   } else {
-    if (valid) code = GammaStep<R, kWoodcock>(s, g, res, T, seed, i, mv, sh.fin.st, (int)threadIdx.x);
+    if (valid) code = GammaStep<R, kWoodcock>(KernelArgs<MoveArgs<R>>().s.t.n, i, mv, sh.fin.st, (int)threadIdx.x);
     SampleBlock<kB, kPConv, kPPE>(sh.fin, code, [&](int j, Staged& r, uint8_t c, int proc) {
+      const MoveArgs<R>& a = KernelArgs<MoveArgs<R>>();
       Trk<R> k;
       Rng rng;
       SecList<R> sl;
       sl.ns = 0;
       const R pe = (R)r.pe;
-      Unstage(r, c, seed, k, rng);
-      GammaFinal(T, k, proc, pe, sl, rng);
-      StoreFinal(t, res, n, i0 + j, k, rng, sl, k.edep, r);
+      Unstage(r, c, a.seed, k, rng);
+      GammaFinal(a.T, k, proc, pe, sl, rng);
+      const MoveArgs<R>& w = KernelArgs<MoveArgs<R>>();
+      StoreFinal(w.s.t, w.res, w.s.t.n, i0 + j, k, rng, sl, k.edep, r);
     });
   }
+  const MoveArgs<R>& a = KernelArgs<MoveArgs<R>>();
+  const Stack& s = a.s;
+  const Slabs& g = a.g;
+  const hepem_tracks& t = s.t;
   __syncthreads();
   const Staged r = sh.fin.st[threadIdx.x];
   __syncthreads();  // the hash table takes the records' place
@@ -583,7 +616,7 @@ __global__ void __launch_bounds__(kB, sizeof(R) == sizeof(double) ? 3 : 4)
       double e = ekin + (t.ptype[i] == 1 && ekin > 0.0 ? 2.0 * kElectronMass : 0.0);
       if (nsec > 0) e += r.dir[1];
       if (nsec > 1) e += r.dir[2];
-      atomicAdd(&leak[ev], (unsigned long long)llrint(e * kFix));
+      atomicAdd(&a.leak[ev], (unsigned long long)llrint(e * kFix));
       alive = false;
       nsec = 0;
     } else if (alive && sd != 0) {
@@ -595,7 +628,7 @@ __global__ void __launch_bounds__(kB, sizeof(R) == sizeof(double) ? 3 : 4)
     // couple's region applies cuts, a secondary below its production
     // threshold is deposited at the step instead of stacked (an e+ with its
     // annihilation energy, when the gamma threshold exceeds the electron mass)
-    const int a = l0 % g.nabs;
+    const int ab = l0 % g.nabs;
     uint32_t mask = 0u;
 #pragma unroll
     for (int sl = 0; sl < 2; ++sl) {
@@ -603,10 +636,10 @@ __global__ void __launch_bounds__(kB, sizeof(R) == sizeof(double) ? 3 : 4)
       const int pt = sl ? (int)r.stream : r.id;
       const double se = sl ? r.dir[2] : r.dir[1];
       bool cut = false;
-      if (g.applyCuts[a]) {
-        if (pt == 0) cut = se < g.cutE[a];
-        else if (pt == 1) cut = kElectronMass < g.cutG[a] && se < g.cutP[a];
-        else cut = se < g.cutG[a];
+      if (g.applyCuts[ab]) {
+        if (pt == 0) cut = se < g.cutE[ab];
+        else if (pt == 1) cut = kElectronMass < g.cutG[ab] && se < g.cutP[ab];
+        else cut = se < g.cutG[ab];
       }
       if (cut) {
         edep += pt == 1 ? se + 2.0 * kElectronMass : se;
@@ -617,7 +650,7 @@ __global__ void __launch_bounds__(kB, sizeof(R) == sizeof(double) ? 3 : 4)
         else ++cE;
       }
     }
-    next[i] = (uint8_t)(mask | (alive ? kSurvives : 0));
+    a.next[i] = (uint8_t)(mask | (alive ? kSurvives : 0));
     if (alive) {
       if (isE) ++cE;
       else ++cG;
@@ -649,18 +682,18 @@ __global__ void __launch_bounds__(kB, sizeof(R) == sizeof(double) ? 3 : 4)
   __syncthreads();
   for (int e = threadIdx.x; e < kHash; e += kB) {
     const unsigned long long k = sh.hash.key[e];
-    if (k != kNone) atomicAdd(&dep[k], sh.hash.val[e]);
+    if (k != kNone) atomicAdd(&a.dep[k], sh.hash.val[e]);
   }
   uint32_t xE, xG, tE, tG, tns;
   hepem::BlockScan2<kB>(cE, cG, ns | (ended << 16), xE, xG, tE, tG, tns);
   if (valid) {
-    offE[i] = xE;
-    offG[i] = xG;
+    a.offE[i] = xE;
+    a.offG[i] = xG;
   }
   if (threadIdx.x == 0) {
-    bsumE[blockIdx.x] = tE;
-    bsumG[blockIdx.x] = tG;
-    bsec[blockIdx.x] = tns;
+    a.bsumE[blockIdx.x] = tE;
+    a.bsumG[blockIdx.x] = tG;
+    a.bsec[blockIdx.x] = tns;
   }
 }
 
@@ -1145,18 +1178,12 @@ extern "C" int hepem_slab_run(const hepem_ctx* ctx, const hepem_slab_setup* su, 
       a.t.n = n;
       // the e-/e+ part of the stack comes first
       const int ge = (ne + kB - 1) / kB, gg = (n - ne + kB - 1) / kB;
-      if (fp64 && woodcock)
-        hipLaunchKernelGGL((k_sh_move<double, true>), dim3(ge + gg), dim3(kB), 0, st, a, g, res, HepemTables64(ctx), seed, ne, ge, dep,
-                           leak, goesOn, offs, offs + cap, bsum, bsum + nblk, bsec);
-      else if (fp64)
-        hipLaunchKernelGGL((k_sh_move<double, false>), dim3(ge + gg), dim3(kB), 0, st, a, g, res, HepemTables64(ctx), seed, ne, ge, dep,
-                           leak, goesOn, offs, offs + cap, bsum, bsum + nblk, bsec);
-      else if (woodcock)
-        hipLaunchKernelGGL((k_sh_move<float, true>), dim3(ge + gg), dim3(kB), 0, st, a, g, res, HepemTables32(ctx), seed, ne, ge, dep,
-                           leak, goesOn, offs, offs + cap, bsum, bsum + nblk, bsec);
-      else
-        hipLaunchKernelGGL((k_sh_move<float, false>), dim3(ge + gg), dim3(kB), 0, st, a, g, res, HepemTables32(ctx), seed, ne, ge, dep,
-                           leak, goesOn, offs, offs + cap, bsum, bsum + nblk, bsec);
+      const auto move = [&](auto kernel, const auto& T) {
+        hipLaunchKernelGGL(kernel, dim3(ge + gg), dim3(kB), 0, st,
+                           {a, g, res, T, seed, ne, ge, dep, leak, goesOn, offs, offs + cap, bsum, bsum + nblk, bsec});
+      };
+      if (fp64) move(woodcock ? k_sh_move<double, true> : k_sh_move<double, false>, HepemTables64(ctx));
+      else move(woodcock ? k_sh_move<float, true> : k_sh_move<float, false>, HepemTables32(ctx));
       r->substeps += ne;
       // primaries of the next events join once the stack runs low, and no
       // sooner after the last ones than the first events took to reach their
