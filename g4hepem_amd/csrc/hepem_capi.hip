@@ -963,9 +963,9 @@ void LaunchStepBatched(const DevTables<R>& T, const hepem_batch_plan* p, uint64_
     hipLaunchKernelGGL((k_step_select_batched_q<R, S>), dim3(p->grid), dim3(ShapeBlock(S)), 0, s, T, seed, p->dDescs,
                        p->dChunkBatch + p->cbOff[S], p->nchunks[S], p->dQueue, p->dCounters, p->dCode, p->dStaged, next);
   else if (TileLocal(p))
-    hipLaunchKernelGGL((k_step_select_local_batched<R>), dim3(p->grid), dim3(kBlock), 0, s, T,
-                       seed, p->dDescs, p->dTileBatch + p->tbOff[kParticleTiles], (int)p->ntiles, p->dQueue, p->dCounters,
-                       p->dLocal, p->dCode, p->dStaged);
+    hipLaunchKernelGGL((k_step_select_local_batched<R>), dim3(p->grid), dim3(kBlock), 0, s,
+                       BatchArgs<R>{T, seed, p->dDescs, p->dTileBatch + p->tbOff[kParticleTiles], (int)p->ntiles, p->dQueue,
+                                    p->dCounters, p->dLocal, p->dCode, p->dStaged});
   else
     hipLaunchKernelGGL((k_step_select_batched<R, S>), dim3(p->grid), dim3(ShapeBlock(S)), 0, s, T, seed, p->dDescs, p->dChunkBatch + p->cbOff[S],
                        p->nchunks[S], p->dQueue, p->dCounters, p->dCode, p->dStaged);

@@ -1188,30 +1188,48 @@ __global__ void __launch_bounds__(kClassifyBlock) k_classify_local_batched(const
 // batch (kBlock threads, a grid of LocalSelectGridTiles(ntiles)): the blocks
 // of the plan's tiles are placed as k_step_select_local places a single
 // batch's, and each records what StepSelectChunk records.
-template <typename R>
-__global__ void __launch_bounds__(kBlock, 4) k_step_select_local_batched(DevTables<R> T, uint64_t seed,
-                                                                      const BatchDev* __restrict__ d,
-                                                                      const uint32_t* __restrict__ tbatch, int ntiles,
-                                                                      const uint32_t* __restrict__ queue,
-                                                                      uint32_t* __restrict__ bcounters,
-                                                                      const uint32_t* __restrict__ ecount,
-                                                                      uint8_t* __restrict__ code, Staged* __restrict__ st) {
-  int tile, chunk;
-  if (!LocalSelectChunk(ntiles, tile, chunk)) return;
-  const int b = __builtin_amdgcn_readfirstlane((int)tbatch[tile]);
-  // by reference: copies would keep 84 scalar registers of pointers alive
-  const hepem_tracks& in = d[b].in;
-  hepem_tracks& out = const_cast<hepem_tracks&>(d[b].out);
-  const hepem_step_out& res = d[b].res;
-  const int n = in.n;
-  const int tile0 = (tile - (int)d[b].tile0) * kClassifyTile;
-  const int m = min(kClassifyTile, n - tile0);
-  const int jl = chunk * kBlock + (int)threadIdx.x;
-  if (jl >= m) return;
-  const uint32_t qoff = d[b].qoff;
-  const int i = (int)queue[qoff + tile0 + jl];
-  code[qoff + i] = StepSelect<R>([&] { return StepView<R>{T, seed, in, out, res, bcounters + 4 * b}; }, n, i, jl < (int)ecount[tile],
-                                 st + qoff, i);
+template <typename R> struct BatchArgs {
+  DevTables<R> T;
+  uint64_t seed;
+  const BatchDev* d;
+  const uint32_t* tbatch;
+  int ntiles;
+  const uint32_t* queue;
+  uint32_t* bcounters;
+  const uint32_t* ecount;
+  uint8_t* code;
+  Staged* st;
+};
+// Descriptor of batch b: constant memory while a kernel runs, so its words are
+// scalar loads wherever they are read.
+template <typename R> HD const BatchDev& Descriptor(int b) {
+  return *(const BatchDev*)((const __attribute__((address_space(4))) BatchDev*)KernelArgs<BatchArgs<R>>().d + b);
+}
+template <typename R> __global__ void __launch_bounds__(kBlock, 4) k_step_select_local_batched(BatchArgs<R>) {
+  int tile, chunk, b, n, i;
+  uint32_t qoff;
+  bool isE;
+  {
+    const BatchArgs<R>& a = KernelArgs<BatchArgs<R>>();
+    if (!LocalSelectChunk(a.ntiles, tile, chunk)) return;
+    b = __builtin_amdgcn_readfirstlane((int)a.tbatch[tile]);
+    const BatchDev& d = Descriptor<R>(b);
+    n = d.in.n;
+    const int tile0 = (tile - (int)d.tile0) * kClassifyTile;
+    const int m = min(kClassifyTile, n - tile0);
+    const int jl = chunk * kBlock + (int)threadIdx.x;
+    if (jl >= m) return;
+    qoff = d.qoff;
+    i = (int)a.queue[qoff + tile0 + jl];
+    isE = jl < (int)a.ecount[tile];
+  }
+  const auto view = [b] {
+    const BatchArgs<R>& a = KernelArgs<BatchArgs<R>>();
+    const BatchDev& d = Descriptor<R>(b);
+    return StepView<R>{a.T, a.seed, d.in, const_cast<hepem_tracks&>(d.out), d.res, a.bcounters + 4 * b};
+  };
+  const uint8_t c = StepSelect<R>(view, n, i, isE, KernelArgs<BatchArgs<R>>().st + qoff, i);
+  KernelArgs<BatchArgs<R>>().code[qoff + i] = c;
 }
 
 // Next work item of a persistent kernel: thread 0 takes it from *next and the
