@@ -12,12 +12,12 @@
 //               the region sets fIsMultipleStepsInMSCTrans and no boundary was
 //               reached, the next sub-step is what is left of the discrete step
 //               (:571-594);
-//   LoopFinish  the loss fluctuation on the summed mean loss from the step's
+//   LoopFinishSelect  the loss fluctuation on the summed mean loss from the step's
 //               pre-step energy (:597-606), then at-rest annihilation or
 //               PerformDiscrete (:611-650; winner 3 resets its interaction
 //               length and draws the delta test, as with a lepto-nuclear process
 //               attached).
-// ElectronSlabStep runs them with the caller's geometry a slab across x.
+// SlabBegin and SlabSubstep run them with the caller's geometry a slab across x.
 #pragma once
 
 #include <cfloat>
@@ -103,9 +103,9 @@ template <typename R> HD bool LoopAlong(const DevTables<R>& T, ElState<R>& el, S
   return sampled;
 }
 
-// LoopFinish up to the final-state sampling of the discrete interaction:
+// The end of the step up to the final-state sampling of the discrete interaction:
 // returns the process whose final state is to be sampled (0 ionisation,
-// 1 brem, 2 annihilation in flight; ElectronFinalState) or -1.
+// 1 brem, 2 annihilation in flight; ElectronProc in dev_final.hh) or -1.
 template <typename R>
 HD int LoopFinishSelect(const DevTables<R>& T, ElState<R>& el, StepLoop<R>& L, SecList<R>& sl, Rng& rng) {
   Trk<R>& t = el.t;
@@ -122,21 +122,6 @@ HD int LoopFinishSelect(const DevTables<R>& T, ElState<R>& el, StepLoop<R>& L, S
   if (L.left) return -1;
   const int proc = ElectronSelectDiscrete(T, t, rng);
   return proc >= 0 && proc < 3 ? proc : -1;
-}
-
-// The final state of the discrete interaction `proc` (PerformDiscrete,
-// G4HepEmElectronManager.icc:443-458).
-template <typename R> HD void ElectronFinalState(const DevTables<R>& T, Trk<R>& t, int proc, SecList<R>& sl, Rng& rng) {
-  switch (proc) {
-    case 0: IoniPerform(T, t, sl, rng); break;
-    case 1: BremPerform(T, t, sl, rng, t.ekin < T.bremModelLim); break;
-    case 2: AnnihilateInFlight(t, sl, rng); break;
-    default: break;
-  }
-}
-
-template <typename R> HD void LoopFinish(const DevTables<R>& T, ElState<R>& el, StepLoop<R>& L, SecList<R>& sl, Rng& rng) {
-  ElectronFinalState(T, el.t, LoopFinishSelect(T, el, L, sl, rng), sl, rng);
 }
 
 // The MSC displacement of a sub-step that did not end on a boundary
@@ -173,7 +158,7 @@ struct SlabPos {
 
 // The slab step in pieces, for callers that interleave the sub-steps of
 // several tracks: SlabBegin, then SlabSubstep until it returns true, then
-// LoopFinishSelect (or LoopFinish).
+// LoopFinishSelect.
 template <typename R> HD void SlabBegin(const DevTables<R>& T, ElState<R>& el, StepLoop<R>& L, Rng& rng, SlabPos& g) {
   Trk<R>& t = el.t;
   t.safety = t.onBoundary ? (R)0.0 : (R)fmax(fmin(g.x - g.lo, g.hi - g.x), 0.0);
@@ -217,21 +202,6 @@ template <typename R> HD bool SlabSubstep(const DevTables<R>& T, ElState<R>& el,
   if (LoopAlong(T, el, L, rng) && !limited) x = DisplaceInSlab(el.msc, x, g.lo, g.hi);
   g.x = x;
   return !L.cont || L.nsub >= kMaxSubsteps;
-}
-
-// ElectronSlabStep up to the final-state sampling: returns the process whose
-// final state is to be sampled (see LoopFinishSelect) or -1.
-template <typename R>
-HD int ElectronSlabStepSelect(const DevTables<R>& T, ElState<R>& el, StepLoop<R>& L, SecList<R>& sl, Rng& rng, SlabPos& g) {
-  SlabBegin(T, el, L, rng, g);
-  while (!SlabSubstep(T, el, L, rng, g)) {
-  }
-  return LoopFinishSelect(T, el, L, sl, rng);
-}
-
-template <typename R>
-HD void ElectronSlabStep(const DevTables<R>& T, ElState<R>& el, StepLoop<R>& L, SecList<R>& sl, Rng& rng, SlabPos& g) {
-  ElectronFinalState(T, el.t, ElectronSlabStepSelect(T, el, L, sl, rng, g), sl, rng);
 }
 
 }  // namespace hepem
