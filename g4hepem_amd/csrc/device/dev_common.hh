@@ -10,6 +10,7 @@
 #include <stdint.h>
 
 #define HD __device__ __forceinline__
+#define HEPEM_INLINE __attribute__((always_inline))  // of a lambda in device code
 
 namespace hepem {
 
@@ -29,7 +30,10 @@ constexpr int kSBGuide = 32;           // buckets of the SB search guide
 // The arguments of a kernel that takes one struct A, to be read where they are
 // used: each call gives an address that the compiler cannot tell from another's,
 // so no argument read before it is held in scalar registers (or spilled from
-// them) past it.
+// them) past it. Only a kernel has the address: in a function that is called it
+// is null. Whatever calls this is therefore inlined into its kernel at every
+// optimisation level (HD, HEPEM_INLINE), and A is the kernel's one parameter
+// (asserted after each of the kernels).
 template <typename A> HD const A& KernelArgs() {
   auto p = __builtin_amdgcn_kernarg_segment_ptr();
 #if defined(__HIP_DEVICE_COMPILE__)

@@ -14,6 +14,8 @@
 // order and are bit-identical to an unsorted pass.
 #pragma once
 
+#include <type_traits>
+
 #include "device/dev_final.hh"
 #include "device/dev_physics.hh"
 #include "device/dev_soa.hh"
@@ -752,10 +754,11 @@ template <typename R> __global__ void __launch_bounds__(kBlock, 4) k_step_select
   bool isE = false, none;
   const int i = StepSlot<R>(isE, none);
   if (i < 0) return;
-  const uint8_t c = StepSelect<R>([] { return ArgsView<R>(); }, KernelArgs<StepArgs<R>>().in.n, i, isE,
+  const uint8_t c = StepSelect<R>([]() HEPEM_INLINE { return ArgsView<R>(); }, KernelArgs<StepArgs<R>>().in.n, i, isE,
                                   KernelArgs<StepArgs<R>>().st, i);
   KernelArgs<StepArgs<R>>().code[i] = c;
 }
+static_assert(std::is_same_v<decltype(k_step_select_local<double>), void(StepArgs<double>)>);
 
 // The whole step in one launch: stage 1 as k_step_select_local, then the final
 // states of the block's pending slots, sorted by process within the block.
@@ -781,14 +784,15 @@ __global__ void __launch_bounds__(kBlock, kStepBlockWaves<R>) k_step_block(StepA
   if (none) return;  // the whole block
   slot[threadIdx.x] = i;
   if (i >= 0)
-    code = StepSelect<R>([] { return ArgsView<R>(); }, KernelArgs<StepArgs<R>>().in.n, i, isE, fin.st, (int)threadIdx.x);
-  SampleBlock<kBlock, kPIoniEl, kPPE>(fin, code, [&](int j, const Staged& r, uint8_t c, int proc) {
+    code = StepSelect<R>([]() HEPEM_INLINE { return ArgsView<R>(); }, KernelArgs<StepArgs<R>>().in.n, i, isE, fin.st, (int)threadIdx.x);
+  SampleBlock<kBlock, kPIoniEl, kPPE>(fin, code, [&](int j, const Staged& r, uint8_t c, int proc) HEPEM_INLINE {
     const StepArgs<R>& a = KernelArgs<StepArgs<R>>();
     hepem_tracks& out = const_cast<hepem_tracks&>(a.out);
     if (proc < kPConv) ElectronInteract<R>(a.T, a.seed, out, a.res, a.in.n, slot[j], r, c);
     else GammaInteract<R>(a.T, a.seed, out, a.res, a.in.n, slot[j], r, c);
   });
 }
+static_assert(std::is_same_v<decltype(k_step_block<double>), void(StepArgs<double>)>);
 
 // Thread -> (slot, is-e-/e+) of the split HowFar and Perform kernels. A
 // mixed batch's queue is read in the layout its hepem_howfar prepare chose
@@ -1223,7 +1227,7 @@ template <typename R> __global__ void __launch_bounds__(kBlock, 4) k_step_select
     i = (int)a.queue[qoff + tile0 + jl];
     isE = jl < (int)a.ecount[tile];
   }
-  const auto view = [b] {
+  const auto view = [b]() HEPEM_INLINE {
     const BatchArgs<R>& a = KernelArgs<BatchArgs<R>>();
     const BatchDev& d = Descriptor<R>(b);
     return StepView<R>{a.T, a.seed, d.in, const_cast<hepem_tracks&>(d.out), d.res, a.bcounters + 4 * b};
@@ -1231,6 +1235,7 @@ template <typename R> __global__ void __launch_bounds__(kBlock, 4) k_step_select
   const uint8_t c = StepSelect<R>(view, n, i, isE, KernelArgs<BatchArgs<R>>().st + qoff, i);
   KernelArgs<BatchArgs<R>>().code[qoff + i] = c;
 }
+static_assert(std::is_same_v<decltype(k_step_select_local_batched<double>), void(BatchArgs<double>)>);
 
 // Next work item of a persistent kernel: thread 0 takes it from *next and the
 // block reads it from LDS (the second barrier keeps thread 0 from overwriting

@@ -31,6 +31,7 @@
 #include <cstring>
 #include <limits>
 #include <new>
+#include <type_traits>
 #include <vector>
 
 #include "device/dev_final.hh"
@@ -563,7 +564,7 @@ __global__ void __launch_bounds__(kB, sizeof(R) == sizeof(double) ? 3 : 4)
   const bool valid = i < last;
   if (isE) {
     if (valid) code = ElectronSubstep<R>(KernelArgs<MoveArgs<R>>().s.t.n, i, mv, sh.fin.st, (int)threadIdx.x);
-    SampleBlock<kB, kPIoniEl, kPAnnih>(sh.fin, code, [&](int j, Staged& r, uint8_t c, int proc) {
+    SampleBlock<kB, kPIoniEl, kPAnnih>(sh.fin, code, [&](int j, Staged& r, uint8_t c, int proc) HEPEM_INLINE {
       const MoveArgs<R>& a = KernelArgs<MoveArgs<R>>();
       Trk<R> k;
       Rng rng;
@@ -577,7 +578,7 @@ __global__ void __launch_bounds__(kB, sizeof(R) == sizeof(double) ? 3 : 4)
     });
   } else {
     if (valid) code = GammaStep<R, kWoodcock>(KernelArgs<MoveArgs<R>>().s.t.n, i, mv, sh.fin.st, (int)threadIdx.x);
-    SampleBlock<kB, kPConv, kPPE>(sh.fin, code, [&](int j, Staged& r, uint8_t c, int proc) {
+    SampleBlock<kB, kPConv, kPPE>(sh.fin, code, [&](int j, Staged& r, uint8_t c, int proc) HEPEM_INLINE {
       const MoveArgs<R>& a = KernelArgs<MoveArgs<R>>();
       Trk<R> k;
       Rng rng;
@@ -696,6 +697,7 @@ __global__ void __launch_bounds__(kB, sizeof(R) == sizeof(double) ? 3 : 4)
     a.bsec[blockIdx.x] = tns;
   }
 }
+static_assert(std::is_same_v<decltype(k_sh_move<double, false>), void(MoveArgs<double>)>);
 
 // In-place exclusive scans of the nb block sums of e-/e+ and gamma slots by
 // one block; the round's secondaries are added to *nsecTotal. The `inject`
