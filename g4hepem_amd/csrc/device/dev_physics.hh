@@ -510,14 +510,15 @@ template <typename R> HD R SampleELossFluctuation(R tcut, R excEner, R meanELoss
       // the Poisson sums' reciprocals: 131k tracks 81.9 us instead of 84.3,
       // 1000 tracks 54 instead of 57).
       int left = nnb;
-      uint32_t nb = (rng.ctr + 1u) >> 1;
+      uint32_t d = rng.ctr + 1u;  // d >> 1: the block of the next draw
       if ((rng.ctr & 1u) && left > 0) {
         eloss += w3 / ((R)1. - w * (R)rng.hold);
         --left;
       }
       while (left > 0) {
         double u0, u1;
-        rng.block(nb++, u0, u1);
+        rng.block(d >> 1, u0, u1);
+        d += 2u;
         eloss += w3 / ((R)1. - w * (R)u0);
         const R next = eloss + w3 / ((R)1. - w * (R)u1);
         eloss = left > 1 ? next : eloss;
@@ -1226,15 +1227,14 @@ template <typename R> HD void SampleNumIALeft(R* nial, Rng& rng) {
   const uint32_t c1 = n0 ? 1u : 0u, c2 = c1 + (n1 ? 1u : 0u), c3 = c2 + (n2 ? 1u : 0u), cnt = c3 + (n3 ? 1u : 0u);
   if (cnt == 0u) return;
   const bool odd = (rng.ctr & 1u) != 0;
-  const uint32_t nb = (rng.ctr + 1u) >> 1;
   double v0, v1;
-  rng.block(nb, v0, v1);
+  rng.block((rng.ctr + 1u) >> 1, v0, v1);
   const R l0 = -vlog((R)(odd ? rng.hold : v0));
   R l1 = l0, l2 = l0, l3 = l0;
   double hold = v1;
   if (cnt > 1u) {
     double w0, w1;
-    rng.block(nb + 1u, w0, w1);
+    rng.block((rng.ctr + 3u) >> 1, w0, w1);
     l1 = -vlog((R)(odd ? v0 : v1));
     l2 = -vlog((R)(odd ? v1 : w0));
     l3 = -vlog((R)(odd ? w0 : w1));
