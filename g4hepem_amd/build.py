@@ -63,11 +63,13 @@ CPP_TEST_DIR = ROOT / "tests" / "cpp"
 # the C++ host-layer test programs: g4hepem_amd.hpp (batches) and
 # g4hepem_amd_onetrack.hpp (the one-track drop-in)
 CPP_TESTS = ("test_managers", "test_onetrack")
+# programs that test the device code itself, compiled as it is
+DEVICE_TESTS = ("test_division",)
 CPP_TEST_BIN = CPP_TEST_DIR / "test_managers"
 
 
 def build_cpp_tests() -> Path:
-    """The C++ host-layer test programs, linked against the in-tree library."""
+    """The C++ host-layer test programs, linked against the in-tree library, and the device-code tests."""
     for name in CPP_TESTS:
         out = CPP_TEST_DIR / name
         tmp = out.with_suffix(".tmp")
@@ -75,6 +77,12 @@ def build_cpp_tests() -> Path:
                "-packed-fp32-ops", f"-I{ROOT / 'include'}", "-o", tmp, CPP_TEST_DIR / f"{name}.cpp", f"-L{PKG}",
                "-lg4hepem_amd", "-Wl,-rpath,$ORIGIN/../../g4hepem_amd"]
         _run(cmd)
+        os.replace(tmp, out)
+    for name in DEVICE_TESTS:
+        out = CPP_TEST_DIR / name
+        tmp = out.with_suffix(".tmp")
+        _run([_hipcc(), *(f for f in HIPCC_FLAGS if f != "-shared"), f"-I{CSRC}", f"-I{ROOT / 'include'}", "-o", tmp,
+              CPP_TEST_DIR / f"{name}.hip"])
         os.replace(tmp, out)
     return CPP_TEST_BIN
 

@@ -49,7 +49,8 @@ template <typename T> HD T tmin(T a, T b) { return a < b ? a : b; }
 // of normal numbers (a may be 0): a reciprocal refined twice and a quotient
 // corrected by its exact remainder. A general division also scales its
 // operands and mends special values, three of its eleven instructions, which
-// never act there.
+// never act there. (-0 / b is +0; compared with the division in
+// tests/cpp/test_division.hip.)
 HD double DivInRange(double a, double b) {
 #if defined(__HIP_DEVICE_COMPILE__)
   double y = __builtin_amdgcn_rcp(b);
@@ -172,8 +173,8 @@ HD uint32_t Xor3(uint32_t a, uint32_t b, uint32_t c) {
 // nearest double (float) r to 1 / n, q = a * r is within 2 ulp, its remainder
 // a - n q is exact (n has at most 5 bits) and q + r (a - n q) is off by less
 // than 2^-45 ulp, while a / n is either representable or at least 1 / (2 n) ulp
-// from a rounding boundary. (Compared on the host: every float mantissa and
-// 10^8 doubles, half of them next to a multiple of n, without a difference.)
+// from a rounding boundary. (tests/cpp/test_division.hip compares every float
+// mantissa and 10^9 doubles, half of them next to a multiple of n.)
 constexpr int kPoissonSmall = 24;
 __constant__ double kRecip[kPoissonSmall + 1] = {0., 1. / 1., 1. / 2., 1. / 3., 1. / 4., 1. / 5., 1. / 6., 1. / 7., 1. / 8.,
   1. / 9., 1. / 10., 1. / 11., 1. / 12., 1. / 13., 1. / 14., 1. / 15., 1. / 16., 1. / 17., 1. / 18., 1. / 19., 1. / 20.,
