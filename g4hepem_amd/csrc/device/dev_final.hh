@@ -126,7 +126,9 @@ template <int NT> struct BlockFinals {
 // in b.st[threadIdx.x]) to the waves, up to 64 of one process at a time, and
 // calls sample(thread, record, code, process) for each. Every thread of the
 // block calls it; codes are of the processes P0..P1. Memory written before the
-// call or by sample is visible to the block after it.
+// call is visible to sample. It ends without a barrier: what sample writes is
+// there for the rest of the block, and b free for another use, only after the
+// caller's next __syncthreads().
 template <int NT, int P0, int P1, typename F>
 __device__ __forceinline__ void SampleBlock(BlockFinals<NT>& b, uint8_t code, F sample) {
   static_assert(NT <= 256, "list entries are 8 bits");
