@@ -637,11 +637,20 @@ extern "C" int hepem_step_prepare(const hepem_ctx* c, const hepem_tracks* in, vo
 
 namespace {
 // The step in one launch (k_step_block) instead of two stages: always in the
-// FP32-table form; in FP64 up to the slots of one resident round of its blocks
-// (256 CUs x 3 blocks): to there it is faster in both orders of the slots (131k
-// mixed 66 us against 75, 200k ordered 79 against 98), and beyond, where a
-// second round begins, slower (262k mixed 111 against 100).
-constexpr int kBlockStepMax64 = 256 * 3 * kBlock;
+// FP32-table form; in FP64 up to the slots of one resident round of its blocks.
+// A step in us, one launch against two stages, kinds interleaved and (e-/e+
+// first), fresh tracks:
+//   131072 slots   66 : 78   ( 71 : 78)
+//   196608         81 : 94   ( 76 : 85)
+//   200003         97 : 96   ( 77 : 86)
+//   262144        120 : 104  ( 87 : 92)
+//   300007        117 : 108  (109 : 100)
+// Interleaved slots lose where the second round begins, and tracks on their way
+// more so (196608 90 : 91, 200003 111 : 100). Slots in kind order gain up to
+// 250k or so, but neither the order nor the kinds are known to the host.
+constexpr int kCUs = 256;
+constexpr int kBlockStepMax64 = kCUs * kStepBlockWaves<double> * kBlock;  // a block is a wave on each SIMD of its CU
+static_assert(kBlock == 4 * 64);
 bool StepsInOneLaunch(const hepem_ctx* c, int n) { return c->precision != HEPEM_FP64 || n <= kBlockStepMax64; }
 }  // namespace
 

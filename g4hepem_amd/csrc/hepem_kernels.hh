@@ -771,8 +771,9 @@ static_assert(std::is_same_v<decltype(k_step_select_local<double>), void(StepArg
 // spills and 1M tracks take 320 us). The FP32-table form runs 5 waves per SIMD
 // (4 VGPRs spilled; left alone it takes 97 VGPRs, 4 waves, and 1M tracks 243 us)
 // and is faster at every size: 16k ordered tracks 44.5 us instead of 50, 1M
-// mixed 225 instead of 260, 3M 588 instead of 756. FP64: 131k 67 instead of 76,
-// 200k 92 and 92, 300k 117 and 108, 1M 309 and 294.
+// mixed 225 instead of 260, 3M 588 instead of 756. FP64 up to one resident
+// round: 131k 66 instead of 78; 1M 309 against 294 (StepsInOneLaunch has both
+// sides of the line).
 template <typename R> constexpr int kStepBlockWaves = sizeof(R) == sizeof(double) ? 3 : 5;
 template <typename R>
 __global__ void __launch_bounds__(kBlock, kStepBlockWaves<R>) k_step_block(StepArgs<R>) {
