@@ -174,7 +174,7 @@ HD uint32_t Xor3(uint32_t a, uint32_t b, uint32_t c) {
 // a - n q is exact (n has at most 5 bits) and q + r (a - n q) is off by less
 // than 2^-45 ulp, while a / n is either representable or at least 1 / (2 n) ulp
 // from a rounding boundary. (tests/cpp/test_division.hip compares every float
-// mantissa and 10^9 doubles, half of them next to a multiple of n.)
+// mantissa and 8 10^8 doubles, half of them next to a multiple of n.)
 constexpr int kPoissonSmall = 24;
 __constant__ double kRecip[kPoissonSmall + 1] = {0., 1. / 1., 1. / 2., 1. / 3., 1. / 4., 1. / 5., 1. / 6., 1. / 7., 1. / 8.,
   1. / 9., 1. / 10., 1. / 11., 1. / 12., 1. / 13., 1. / 14., 1. / 15., 1. / 16., 1. / 17., 1. / 18., 1. / 19., 1. / 20.,

@@ -1,7 +1,8 @@
 // hepem_kernels.hh -- kernels of the stepping library (one translation unit,
 // included by hepem_capi.hip).
 //
-// Stepping is split in two launches:
+// The step without the process sort is two launches (the sorted forms are
+// described where they stand, below):
 //   k_classify  compaction of track slots by particle type into one queue:
 //               e-/e+ slots fill it from the front, gamma slots from the back
 //               (wave ballots and an LDS scan per tile of kClassifyTile slots,
@@ -402,10 +403,10 @@ __global__ void __launch_bounds__(kBlock) k_el_end(DevTables<R> T, uint64_t seed
 // the interaction lengths and the mean free paths would otherwise hold about 30
 // VGPRs through the MSC and fluctuation sampling. Of the interaction lengths
 // the winner's alone waits (a discrete interaction resets it). Measured: the
-// split Perform's first stage 164 -> 122 VGPRs (4 waves per SIMD instead of 3),
-// the step's 140 -> 135; held to 128 (8 spill accesses outside the loops) it
-// runs 4 waves too: 3M ordered tracks 765 us instead of 800, 300k split calls
-// 162 instead of 169, 1M mixed tracks 314 instead of 318.
+// split Perform's first stage 164 -> 122 VGPRs (4 waves per SIMD instead of 3;
+// 118 by now), the step's 140 -> 135, and held to 128 it runs 4 waves too (by
+// now 125 and nothing spills: ArgsView): 3M ordered tracks 765 us instead of
+// 800, 300k split calls 162 instead of 169, 1M mixed tracks 314 instead of 318.
 template <typename R>
 HD uint8_t ElectronSelectAfterHowFar(const DevTables<R>& T, ElState<R>& el, Rng& rng, const hepem_tracks& in,
                                      hepem_tracks& out, const hepem_step_out& res, int n, int i, Staged* st, int j) {
@@ -588,8 +589,8 @@ HD void GammaInteract(const DevTables<R>& T, uint64_t seed, hepem_tracks& out, c
 // k_classify_tiles lays the pending slots of each tile of kClassifyTile
 // slots out process by process, within the tile's own range of `tlist` (tile
 // offsets, 16 bits), and writes the tile's process offsets and chunk counts
-// to `tinfo` (wave ballots and an LDS scan; no atomics, so the layout is
-// deterministic).
+// to `tinfo` (packed scans over a wave and over the waves' totals; no atomics, so
+// the layout is deterministic).
 //
 // k_interact_tiles gives each wave one chunk of up to 64 entries of one
 // process. A tile's chunks are spread over kInteractParts blocks that go to
